@@ -129,6 +129,23 @@ int rwkv7_wkv_train_backward(int dtype, int64_t B, int64_t T, int64_t H, const v
                              const float *sa, const float *ds_in, void *dr, void *dw,
                              void *dk, void *dv, void *da, void *db, float *ds0,
                              void *stream);
+/*
+ * rwkv7_wkv_train_backward_chunked: the same gradients in 32-token chunks on the
+ * matrix cores, split over the sequence when B x H is below the CU count.
+ * start_known != 0: s0 (nullable: zero) is the forward's initial state; 0: it is
+ * recovered from the first checkpoint, as above.  ws: float32 workspace of
+ * rwkv7_wkv_train_backward_ws_floats floats (may be 0 and ws NULL), 16-byte
+ * aligned.  Tensors not aligned to 4 elements run token by token.
+ */
+int64_t rwkv7_wkv_train_backward_ws_floats(int64_t B, int64_t T, int64_t H);
+int rwkv7_wkv_train_backward_chunked(int dtype, int64_t B, int64_t T, int64_t H,
+                                     const void *r, const void *w, const void *k,
+                                     const void *v, const void *a, const void *b,
+                                     const void *dy, const float *ckpt, const float *sa,
+                                     const float *ds_in, const float *s0, int start_known,
+                                     void *dr, void *dw, void *dk, void *dv, void *da,
+                                     void *db, float *ds0, float *ws, int64_t ws_floats,
+                                     void *stream);
 
 /* ------------------------------------------------------------------------
  * Layer kernels of the stateful model forward.  They replace the eager torch

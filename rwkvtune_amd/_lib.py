@@ -35,6 +35,9 @@ SIGNATURES = {
     "rwkv7_wkv_train_ckpt_floats": (_I64, [_I64, _I64, _I64]),
     "rwkv7_wkv_train_forward": (_I32, [_I32, _I64, _I64, _I64] + [_P] * 11 + [_P]),
     "rwkv7_wkv_train_backward": (_I32, [_I32, _I64, _I64, _I64] + [_P] * 17 + [_P]),
+    "rwkv7_wkv_train_backward_ws_floats": (_I64, [_I64, _I64, _I64]),
+    "rwkv7_wkv_train_backward_chunked": (_I32, [_I32, _I64, _I64, _I64] + [_P] * 11 + [_I32] + [_P] * 8
+                                         + [_I64, _P]),
     "rwkv7_shift_mix": (_I32, [_I32, _I64, _I64, _P, _P, _I32, _I64, _P, _P, _I64, _P, _P, _P, _P, _P, _P,
                                _I64, _P, _P, _I32, _P, _P, _P]),
     "rwkv7_final_norm": (_I32, [_I32, _I64, _I64, _P, _P, _I32, _I64, _P, _P, _P, _P, _P]),

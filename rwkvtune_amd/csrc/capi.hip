@@ -548,6 +548,13 @@ hipError_t launch_wkv7_train_bwd(int B, int T, int H, const void* r, const void*
                                  const void* a, const void* b, const void* dy, const float* ckpt, const float* sa,
                                  const float* ds_in, void* dr, void* dw, void* dk, void* dv, void* da, void* db,
                                  float* ds0, hipStream_t st);
+int64_t wkv7_train_bwd_chunk_ws(int B, int T, int H);
+template <typename IO>
+hipError_t launch_wkv7_train_bwd_chunk(int B, int T, int H, const void* r, const void* w, const void* k,
+                                       const void* v, const void* a, const void* b, const void* dy,
+                                       const float* ckpt, const float* sa, const float* ds_in, const float* s0,
+                                       int start_known, void* dr, void* dw, void* dk, void* dv, void* da, void* db,
+                                       float* ds0, float* ws, hipStream_t st);
 template <typename IO>
 hipError_t launch_wkv7_chunk_train(int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
                                    const void* a, const void* b, void* y, const float* s0, float* s_out, float* ckpt,
@@ -618,6 +625,43 @@ extern "C" int rwkv7_wkv_train_backward(int dtype, int64_t B, int64_t T, int64_t
     RWKV7_DISPATCH(dtype, (launch_wkv7_train_bwd<IO>((int)B, (int)T, (int)H, r, w, k, v, a, b, dy, ckpt, sa, ds_in,
                                                      dr, dw, dk, dv, da, db, ds0, (hipStream_t)stream)));
     return launch_status(e, "wkv7_train_bwd_kernel");
+}
+
+extern "C" int64_t rwkv7_wkv_train_backward_ws_floats(int64_t B, int64_t T, int64_t H) {
+    if (train_sizes("rwkv7_wkv_train_backward_ws_floats", B, T, H) != RWKV7_OK) return -1;
+    ok();
+    if (B == 0 || T == 0) return 0;
+    return wkv7_train_bwd_chunk_ws((int)B, (int)T, (int)H);
+}
+
+extern "C" int rwkv7_wkv_train_backward_chunked(int dtype, int64_t B, int64_t T, int64_t H, const void* r,
+                                                const void* w, const void* k, const void* v, const void* a,
+                                                const void* b, const void* dy, const float* ckpt, const float* sa,
+                                                const float* ds_in, const float* s0, int start_known, void* dr,
+                                                void* dw, void* dk, void* dv, void* da, void* db, float* ds0,
+                                                float* ws, int64_t ws_floats, void* stream) {
+    // tensors that the 4-element loads and stores cannot take run token by token, as do rows too long for
+    // 32-bit offsets within a chunk; so do the empty and the invalid calls (the same checks)
+    if (!dtype_ok(dtype) || B <= 0 || T <= 0 || H > (1 << 17) || misaligned(dtype, nullptr, r, w, k, v, a, b) ||
+        misaligned(dtype, nullptr, dr, dw, dk, dv, da, db) || misaligned(dtype, nullptr, dy, dy, dy, dy, dy, dy) ||
+        f32_misaligned(sa) || f32_misaligned(s0))
+        return rwkv7_wkv_train_backward(dtype, B, T, H, r, w, k, v, a, b, dy, ckpt, sa, ds_in, dr, dw, dk, dv, da,
+                                        db, ds0, stream);
+    if (train_sizes("rwkv7_wkv_train_backward_chunked", B, T, H) != RWKV7_OK) return RWKV7_ERR_INVALID;
+    if (any_null(r, w, k, v, a, b, dy, ckpt) || !sa || any_null(dr, dw, dk, dv, da, db, sa, ckpt))
+        return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_train_backward_chunked: null pointer");
+    if (f32_misaligned(ckpt) || f32_misaligned(ds0) || f32_misaligned(ws))
+        return fail(RWKV7_ERR_INVALID,
+                    "rwkv7_wkv_train_backward_chunked: checkpoints, ds0 and ws must be 16-byte aligned");
+    const int64_t need = wkv7_train_bwd_chunk_ws((int)B, (int)T, (int)H);
+    if (need > 0 && (ws == nullptr || ws_floats < need))
+        return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_train_backward_chunked: needs %lld workspace floats, got %lld",
+                    (long long)need, (long long)(ws == nullptr ? 0 : ws_floats));
+    hipError_t e;
+    RWKV7_DISPATCH(dtype, (launch_wkv7_train_bwd_chunk<IO>((int)B, (int)T, (int)H, r, w, k, v, a, b, dy, ckpt, sa,
+                                                           ds_in, s0, start_known, dr, dw, dk, dv, da, db, ds0, ws,
+                                                           (hipStream_t)stream)));
+    return launch_status(e, "wkv7_train_bwd_chunk_kernel");
 }
 
 // ---------------------------------------------------------------------------

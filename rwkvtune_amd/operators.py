@@ -159,15 +159,19 @@ def _train_forward(w, q, k, v, a, b, s0=None, s_out=None):
     return y, ckpt, sa
 
 
-def _train_backward(w, q, k, v, a, b, dy, ckpt, sa, ds_in=None, want_ds0=False):
+def _train_backward(w, q, k, v, a, b, dy, ckpt, sa, ds_in=None, want_ds0=False, s0=None, start_known=False):
+    """``start_known``: ``s0`` (None: zero) is the forward's initial state; otherwise
+    it is recovered from the first checkpoint."""
     B, T, H, N = q.shape
+    need = _lib.load().rwkv7_wkv_train_backward_ws_floats(B, T, H)
+    ws = torch.empty(need, dtype=torch.float32, device=q.device) if need > 0 else None
     grads = [torch.empty_like(x) for x in (w, q, k, v, a, b)]
     dw, dq, dk, dv, da, db = grads
     ds0 = torch.empty((B, H, N, N), dtype=torch.float32, device=q.device) if want_ds0 else None
     P = _lib.ptr
-    _lib.call("rwkv7_wkv_train_backward", _lib.dtype_code(q.dtype), B, T, H, P(q), P(w), P(k), P(v), P(a), P(b),
-              P(dy), P(ckpt), P(sa), P(ds_in), P(dq), P(dw), P(dk), P(dv), P(da), P(db), P(ds0),
-              _lib.stream_of(q))
+    _lib.call("rwkv7_wkv_train_backward_chunked", _lib.dtype_code(q.dtype), B, T, H, P(q), P(w), P(k), P(v), P(a),
+              P(b), P(dy), P(ckpt), P(sa), P(ds_in), P(s0), int(start_known), P(dq), P(dw), P(dk), P(dv), P(da),
+              P(db), P(ds0), P(ws), max(need, 0), _lib.stream_of(q))
     return dw, dq, dk, dv, da, db, ds0
 
 
@@ -192,7 +196,7 @@ class WindBackstepping(torch.autograd.Function):
         assert dy.dtype == torch.bfloat16
         dy = dy.contiguous()
         w, q, k, v, z, b, ckpt, sa = ctx.saved_tensors
-        dw, dq, dk, dv, dz, db, _ = _train_backward(w, q, k, v, z, b, dy, ckpt, sa)
+        dw, dq, dk, dv, dz, db, _ = _train_backward(w, q, k, v, z, b, dy, ckpt, sa, start_known=True)
         return dw, dq, dk, dv, dz, db
 
 
@@ -247,7 +251,8 @@ class WKV7InfctxFunction(torch.autograd.Function):
         dy = dy.contiguous()
         ds_in = None if dstate_out is None else dstate_out.to(torch.float32).contiguous()
         _, ckpt, sa = _train_forward(w, q, k, v, a, b, s0=s0)
-        dw, dq, dk, dv, da, db, ds0 = _train_backward(w, q, k, v, a, b, dy, ckpt, sa, ds_in=ds_in, want_ds0=True)
+        dw, dq, dk, dv, da, db, ds0 = _train_backward(w, q, k, v, a, b, dy, ckpt, sa, ds_in=ds_in, want_ds0=True,
+                                                      s0=s0, start_known=True)
         return dw, dq, dk, dv, da, db, ds0
 
 
@@ -284,7 +289,8 @@ class _InfctxModule:
     def backward(w, q, k, v, a, b, dy, s0, ds_in, dw, dq, dk, dv, da, db, ds):
         ds_in = ds_in if (ds_in is not None and ds_in.numel() > 0) else None
         _, ckpt, sa = _train_forward(w, q, k, v, a, b, s0=s0)
-        g = _train_backward(w, q, k, v, a, b, dy.contiguous(), ckpt, sa, ds_in=ds_in, want_ds0=True)
+        g = _train_backward(w, q, k, v, a, b, dy.contiguous(), ckpt, sa, ds_in=ds_in, want_ds0=True, s0=s0,
+                            start_known=True)
         for dst, src in zip((dw, dq, dk, dv, da, db, ds), g):
             dst.copy_(src)
 
