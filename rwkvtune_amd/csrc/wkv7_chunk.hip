@@ -550,6 +550,11 @@ __device__ __forceinline__ float quad_bcast(float x, int e) {
     }
 }
 
+// Block barrier for data exchanged through LDS.  __syncthreads() also waits for every global load and store
+// of the wave: the loads issued a chunk ahead, y and the training checkpoints.  Training forward at
+// B = 8, T = 4096, H = 32 (bf16, one block per CU): 0.88 -> 0.73 ms; prefill the same either way.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // hi / lo bf16 parts of one value (hardware round-to-nearest-even)
 __device__ __forceinline__ void split1(float x, uint16_t& hi, uint16_t& lo) {
     uint32_t h, l;
@@ -596,7 +601,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         if (nseq <= 256) {
             int* lens = sm.u.lens;
             for (int c = tid; c < nseq; c += 256) lens[c] = cu_seqlens[c + 1] - cu_seqlens[c];
-            __syncthreads();
+            lds_barrier();
             for (int c = tid; c < nseq; c += 256) {
                 const int len = lens[c];
                 int rank = 0;
@@ -606,7 +611,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 }
                 if (rank == s) sm.pick = c;
             }
-            __syncthreads();
+            lds_barrier();
             s = sm.pick;
         }
     }
@@ -719,7 +724,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         if (g == 3) *reinterpret_cast<f32x4*>(&sm.tot[wave][j0]) = inc;
         const bool wave_slow = __ballot(slow) != 0;
         if (lane == 0) sm.slow[wave] = wave_slow ? 1 : 0;
-        __syncthreads();
+        lds_barrier();
         const int4 sl = *reinterpret_cast<const int4*>(sm.slow);
         const bool any_slow = (sl.x | sl.y | sl.z | sl.w) != 0;
 
@@ -800,12 +805,12 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
 
         if (any_slow) {
             // ---- exact token-serial update on a float32 copy of the state in LDS ----
             tile_io(&sm.u.Sf[0][0], SP, true);
-            __syncthreads();
+            lds_barrier();
             const int i = tid >> 2, q = tid & 3;
             for (int t = 0; t < n; ++t) {
                 const size_t off = (size_t)(t0 + t) * C + h * NH;
@@ -836,7 +841,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                     }
                 }
             }
-            __syncthreads();
+            lds_barrier();
             // back to the registers, and the hi/lo planes
             tile_io(&sm.u.Sf[0][0], SP, false);
             store_state_planes(&sm.Sp[0][0][0], ir_t, jt_t, tile, lane);
@@ -844,6 +849,10 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             // the next chunk writes the region that holds Sf after its first barrier
             continue;
         }
+
+        // the raw registers are free from here to the next phase A: fetch the next chunk (LDS barriers do not
+        // wait for global loads, so these stay in flight through phases B to D)
+        if (t0 + L < te) fetch(t0 + L);
 
         // ---- B: two 32x32 tiles per wave, K = 64 over keys, sharing one operand:
         //   wave 0: X (value tile 0) and A_ab,   wave 1: X (value tile 1) and A_ak,
@@ -875,7 +884,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 c1[q] = keep ? c1[q] : 0.f;
             }
             // the products overwrite the planes they were computed from
-            __syncthreads();
+            lds_barrier();
             if (wave == 0) {
                 float* AT = &sm.u.pb.AT[0][0];
 #pragma unroll
@@ -888,7 +897,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 store_planes_T(out, TQ, T32_PLANE, 0, 0, c1, lane);
             }
         }
-        __syncthreads();
+        lds_barrier();
 
         // ---- C: X += V^T A_ak (waves 0/1), stored as X^T; Y += V^T B_rk (waves 2/3) --
         {
@@ -909,7 +918,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 *reinterpret_cast<f32x4*>(XT + xtswz(t, 32 * wave + 8 * g + 4 * (lane >> 5))) =
                     f32x4{accXY[4 * g], accXY[4 * g + 1], accXY[4 * g + 2], accXY[4 * g + 3]};
         }
-        __syncthreads();
+        lds_barrier();
 
         // ---- triangular solve: SA[i][t] = X[i][t] + sum_{u<t} SA[i][u] A_ab[u][t] -----
         // Right-looking: lane q of row i keeps running sums for its targets t = 4m + q.
@@ -984,12 +993,10 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                     if (4 * m + q < n) sa_out[(size_t)(t0 + 4 * m + q) * C + h * NH + i] = pq[m];
             }
         }
-        __syncthreads();
+        lds_barrier();
 
         // ---- D: every wave: its state tile += (b^^T SA)^T, scaled by D_L and stored as the next chunk's
         //         planes; waves 2/3 also Y += SA B_rb (value tile wave - 2) and store y
-        // the raw registers are free from here to the next phase A: fetch the next chunk
-        if (t0 + L < te) fetch(t0 + L);
         const uint16_t* SA = &sm.u.pb.SA[0][0][0];
         auto d_step = [&](int k0) {  // tokens k0 .. k0 + 15 of b^^T SA
             const bf16x8_t sa0 = fragSA(SA, 32 * ir_t, k0, lane), sa1 = fragSA(SA + SA_PLANE, 32 * ir_t, k0, lane);
