@@ -98,6 +98,31 @@ int rwkv7_wkv_prefill(int dtype, int64_t nseq, int64_t H, int64_t total_tokens,
                       void *stream);
 
 /*
+ * The same three calls with a float32 workspace (16-byte aligned; NULL or smaller
+ * than rwkv7_wkv_segment_ws_floats: as without).  With it, 16-bit inputs of few
+ * (sequence, head) pairs are walked in segments side by side instead of one block
+ * per pair: the state recurrence of every segment first, then a scan over the
+ * segments, then the full pass.  ragged = 0: nseq sequences of T tokens.
+ */
+int64_t rwkv7_wkv_segment_ws_floats(int dtype, int64_t nseq, int64_t H, int64_t T,
+                                    int64_t total_tokens, int ragged);
+int rwkv7s_forward_ws(int dtype, int64_t B, int64_t T, int64_t C, int64_t H, float *state,
+                      const void *r, const void *w, const void *k, const void *v,
+                      const void *a, const void *b, void *y, float *ws,
+                      int64_t ws_floats, void *stream);
+int rwkv7_wkv_prefill_ws(int dtype, int64_t nseq, int64_t H, int64_t total_tokens,
+                         const int32_t *cu_seqlens, const int32_t *slot_idx,
+                         float *state_pool, int64_t pool_slots, const void *r,
+                         const void *w, const void *k, const void *v, const void *a,
+                         const void *b, void *y, int chunk_len, float *ws,
+                         int64_t ws_floats, void *stream);
+int rwkv7_wkv_train_forward_ws(int dtype, int64_t B, int64_t T, int64_t H, const void *r,
+                               const void *w, const void *k, const void *v,
+                               const void *a, const void *b, void *y, const float *s0,
+                               float *s_out, float *ckpt, float *sa, float *ws,
+                               int64_t ws_floats, void *stream);
+
+/*
  * Training operator: replaces torch.ops.wind_backstepping.forward / backward
  * (rwkvtune/models/rwkv7/operators/cuda/wkv7_op.cpp:6-18, kernels
  * wkv7_cuda.cu:10-142) and, with s0 / ds_in / ds0, the infinite-context op

@@ -32,6 +32,10 @@ SIGNATURES = {
     "rwkv7s_forward": (_I32, [_I32, _I64, _I64, _I64, _I64] + [_P] * 8 + [_P]),
     "rwkv7_wkv_decode": (_I32, [_I32, _I64, _I64, _P, _I64, _P] + [_P] * 7 + [_P]),
     "rwkv7_wkv_prefill": (_I32, [_I32, _I64, _I64, _I64, _P, _P, _P, _I64] + [_P] * 7 + [_I32, _P]),
+    "rwkv7_wkv_segment_ws_floats": (_I64, [_I32, _I64, _I64, _I64, _I64, _I32]),
+    "rwkv7s_forward_ws": (_I32, [_I32, _I64, _I64, _I64, _I64] + [_P] * 9 + [_I64, _P]),
+    "rwkv7_wkv_prefill_ws": (_I32, [_I32, _I64, _I64, _I64, _P, _P, _P, _I64] + [_P] * 7 + [_I32, _P, _I64, _P]),
+    "rwkv7_wkv_train_forward_ws": (_I32, [_I32, _I64, _I64, _I64] + [_P] * 12 + [_I64, _P]),
     "rwkv7_wkv_train_ckpt_floats": (_I64, [_I64, _I64, _I64]),
     "rwkv7_wkv_train_forward": (_I32, [_I32, _I64, _I64, _I64] + [_P] * 11 + [_P]),
     "rwkv7_wkv_train_backward": (_I32, [_I32, _I64, _I64, _I64] + [_P] * 17 + [_P]),

@@ -16,7 +16,9 @@ hipError_t launch_wkv7_seq(int nseq, int H, int T_uniform, const int32_t* cu_seq
 template <typename IO>
 hipError_t launch_wkv7_chunk(int nseq, int H, int T_uniform, const int32_t* cu_seqlens, const int32_t* slot_idx,
                              int pool_slots, int total_tokens, float* state, const void* r, const void* w,
-                             const void* k, const void* v, const void* a, const void* b, void* y, hipStream_t stream);
+                             const void* k, const void* v, const void* a, const void* b, void* y, float* ws,
+                             int64_t ws_floats, hipStream_t stream);
+int64_t wkv7_chunk_ws(int nseq, int H, int T_uniform, bool ragged, int total, bool two_per_cu);
 
 namespace {
 
@@ -70,24 +72,26 @@ int seq_dispatch(int dtype, int nseq, int H, int T_uniform, const int32_t* cu, c
 
 int chunk_dispatch(int dtype, int nseq, int H, int T_uniform, const int32_t* cu, const int32_t* slot, int pool_slots,
                    int total, float* state, const void* r, const void* w, const void* k, const void* v,
-                   const void* a, const void* b, void* y, hipStream_t st) {
+                   const void* a, const void* b, void* y, float* ws, int64_t ws_floats, hipStream_t st) {
     hipError_t e;
     switch (dtype) {
         case RWKV7_DTYPE_F32:
             e = launch_wkv7_chunk<float>(nseq, H, T_uniform, cu, slot, pool_slots, total, state, r, w, k, v, a, b, y,
-                                         st);
+                                         ws, ws_floats, st);
             break;
         case RWKV7_DTYPE_F16:
             e = launch_wkv7_chunk<f16_t>(nseq, H, T_uniform, cu, slot, pool_slots, total, state, r, w, k, v, a, b, y,
-                                         st);
+                                         ws, ws_floats, st);
             break;
         default:
             e = launch_wkv7_chunk<bf16_t>(nseq, H, T_uniform, cu, slot, pool_slots, total, state, r, w, k, v, a, b,
-                                          y, st);
+                                          y, ws, ws_floats, st);
             break;
     }
     return launch_status(e, "wkv7_chunk_kernel");
 }
+
+bool f32_misaligned(const float* p) { return (((uintptr_t)p) & 15) != 0; }
 
 bool any_null(const void* p0, const void* p1, const void* p2, const void* p3, const void* p4,
               const void* p5, const void* p6, const void* p7) {
@@ -109,9 +113,26 @@ extern "C" int rwkv7_abi_version(void) { return 2; }
 
 extern "C" const char* rwkv7_last_error(void) { return g_err; }
 
+extern "C" int64_t rwkv7_wkv_segment_ws_floats(int dtype, int64_t nseq, int64_t H, int64_t T, int64_t total_tokens,
+                                               int ragged) {
+    ok();
+    if (!dtype_ok(dtype) || dtype == RWKV7_DTYPE_F32 || nseq <= 0 || H <= 0 || total_tokens <= 0 ||
+        (ragged == 0 && T <= 0) || nseq * H > kMaxInt || T > kMaxInt || total_tokens > kMaxInt)
+        return 0;  // sizes that the call itself refuses or that have nothing to split
+    return wkv7_chunk_ws((int)nseq, (int)H, ragged ? 0 : (int)T, ragged != 0, (int)total_tokens,
+                         dtype == RWKV7_DTYPE_BF16);
+}
+
 extern "C" int rwkv7s_forward(int dtype, int64_t B, int64_t T, int64_t C, int64_t H, float* state,
                               const void* r, const void* w, const void* k, const void* v,
                               const void* a, const void* b, void* y, void* stream) {
+    return rwkv7s_forward_ws(dtype, B, T, C, H, state, r, w, k, v, a, b, y, nullptr, 0, stream);
+}
+
+extern "C" int rwkv7s_forward_ws(int dtype, int64_t B, int64_t T, int64_t C, int64_t H, float* state,
+                                 const void* r, const void* w, const void* k, const void* v,
+                                 const void* a, const void* b, void* y, float* ws, int64_t ws_floats,
+                                 void* stream) {
     if (!dtype_ok(dtype)) return fail(RWKV7_ERR_INVALID, "rwkv7s_forward: bad dtype code %d", dtype);
     if (B < 0 || T < 0 || H <= 0) return fail(RWKV7_ERR_INVALID, "rwkv7s_forward: bad sizes B=%lld T=%lld H=%lld",
                                               (long long)B, (long long)T, (long long)H);
@@ -122,13 +143,13 @@ extern "C" int rwkv7s_forward(int dtype, int64_t B, int64_t T, int64_t C, int64_
     if (B * T > kMaxInt || 4 * B * H > kMaxInt || B * T * C > (int64_t)1 << 40)
         return fail(RWKV7_ERR_INVALID, "rwkv7s_forward: problem too large");
     if (any_null(state, r, w, k, v, a, b, y)) return fail(RWKV7_ERR_INVALID, "rwkv7s_forward: null pointer");
-    if (misaligned(dtype, state, r, w, k, v, a, b))
+    if (misaligned(dtype, state, r, w, k, v, a, b) || f32_misaligned(ws))
         return fail(RWKV7_ERR_INVALID, "rwkv7s_forward: inputs must be aligned to 4 elements, the state to 16 bytes");
     hipStream_t st = (hipStream_t)stream;
     if (T == 1)
         return seq_dispatch(dtype, (int)B, (int)H, 1, nullptr, nullptr, (int)B, (int)B, state, r, w, k, v, a, b, y, st);
     return chunk_dispatch(dtype, (int)B, (int)H, (int)T, nullptr, nullptr, (int)B, (int)(B * T), state, r, w, k, v, a,
-                          b, y, st);
+                          b, y, ws, ws_floats, st);
 }
 
 extern "C" int rwkv7_wkv_decode(int dtype, int64_t B, int64_t H, float* state_pool, int64_t pool_slots,
@@ -154,6 +175,15 @@ extern "C" int rwkv7_wkv_prefill(int dtype, int64_t nseq, int64_t H, int64_t tot
                                  int64_t pool_slots, const void* r, const void* w, const void* k,
                                  const void* v, const void* a, const void* b, void* y, int chunk_len,
                                  void* stream) {
+    return rwkv7_wkv_prefill_ws(dtype, nseq, H, total_tokens, cu_seqlens, slot_idx, state_pool, pool_slots, r, w, k,
+                                v, a, b, y, chunk_len, nullptr, 0, stream);
+}
+
+extern "C" int rwkv7_wkv_prefill_ws(int dtype, int64_t nseq, int64_t H, int64_t total_tokens,
+                                    const int32_t* cu_seqlens, const int32_t* slot_idx, float* state_pool,
+                                    int64_t pool_slots, const void* r, const void* w, const void* k,
+                                    const void* v, const void* a, const void* b, void* y, int chunk_len,
+                                    float* ws, int64_t ws_floats, void* stream) {
     if (!dtype_ok(dtype)) return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_prefill: bad dtype code %d", dtype);
     if (nseq < 0 || H <= 0 || total_tokens < 0 || pool_slots < 0)
         return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_prefill: bad sizes");
@@ -166,13 +196,13 @@ extern "C" int rwkv7_wkv_prefill(int dtype, int64_t nseq, int64_t H, int64_t tot
     if (4 * nseq * H > kMaxInt || total_tokens > kMaxInt || pool_slots > kMaxInt)
         return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_prefill: too large");
     if (any_null(state_pool, r, w, k, v, a, b, y)) return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_prefill: null pointer");
-    if (misaligned(dtype, state_pool, r, w, k, v, a, b))
+    if (misaligned(dtype, state_pool, r, w, k, v, a, b) || f32_misaligned(ws))
         return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_prefill: inputs must be aligned to 4 elements, the state to 16 bytes");
     if (chunk_len == 1)
         return seq_dispatch(dtype, (int)nseq, (int)H, 0, cu_seqlens, slot_idx, (int)pool_slots, (int)total_tokens,
                             state_pool, r, w, k, v, a, b, y, (hipStream_t)stream);
     return chunk_dispatch(dtype, (int)nseq, (int)H, 0, cu_seqlens, slot_idx, (int)pool_slots, (int)total_tokens,
-                          state_pool, r, w, k, v, a, b, y, (hipStream_t)stream);
+                          state_pool, r, w, k, v, a, b, y, ws, ws_floats, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -558,7 +588,7 @@ hipError_t launch_wkv7_train_bwd_chunk(int B, int T, int H, const void* r, const
 template <typename IO>
 hipError_t launch_wkv7_chunk_train(int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
                                    const void* a, const void* b, void* y, const float* s0, float* s_out, float* ckpt,
-                                   float* sa, hipStream_t stream);
+                                   float* sa, float* ws, int64_t ws_floats, hipStream_t stream);
 
 namespace {
 int train_sizes(const char* fn, int64_t B, int64_t T, int64_t H) {
@@ -569,7 +599,6 @@ int train_sizes(const char* fn, int64_t B, int64_t T, int64_t H) {
         return fail(RWKV7_ERR_INVALID, "%s: problem too large", fn);
     return RWKV7_OK;
 }
-bool f32_misaligned(const float* p) { return (((uintptr_t)p) & 15) != 0; }
 }  // namespace
 
 extern "C" int64_t rwkv7_wkv_train_ckpt_floats(int64_t B, int64_t T, int64_t H) {
@@ -581,23 +610,30 @@ extern "C" int64_t rwkv7_wkv_train_ckpt_floats(int64_t B, int64_t T, int64_t H) 
 extern "C" int rwkv7_wkv_train_forward(int dtype, int64_t B, int64_t T, int64_t H, const void* r, const void* w,
                                        const void* k, const void* v, const void* a, const void* b, void* y,
                                        const float* s0, float* s_out, float* ckpt, float* sa, void* stream) {
+    return rwkv7_wkv_train_forward_ws(dtype, B, T, H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa, nullptr, 0, stream);
+}
+
+extern "C" int rwkv7_wkv_train_forward_ws(int dtype, int64_t B, int64_t T, int64_t H, const void* r, const void* w,
+                                       const void* k, const void* v, const void* a, const void* b, void* y,
+                                       const float* s0, float* s_out, float* ckpt, float* sa, float* ws,
+                                          int64_t ws_floats, void* stream) {
     if (!dtype_ok(dtype)) return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_train_forward: bad dtype code %d", dtype);
     if (train_sizes("rwkv7_wkv_train_forward", B, T, H) != RWKV7_OK) return RWKV7_ERR_INVALID;
     if (B == 0 || T == 0) return ok();
     if (any_null(r, w, k, v, a, b, y, ckpt) || !sa)
         return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_train_forward: null pointer");
-    if (f32_misaligned(ckpt) || f32_misaligned(s0) || f32_misaligned(s_out))
+    if (f32_misaligned(ckpt) || f32_misaligned(s0) || f32_misaligned(s_out) || f32_misaligned(ws))
         return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_train_forward: checkpoints and states must be 16-byte aligned");
     hipError_t e;
     // 16-bit inputs aligned to 4 elements run the chunked kernel (32-token matrix
     // form on the matrix cores); float32 inputs keep the token-serial kernel
     if (dtype != RWKV7_DTYPE_F32 && B * T <= kMaxInt && !misaligned(dtype, nullptr, r, w, k, v, a, b)) {
         if (dtype == RWKV7_DTYPE_F16)
-            e = launch_wkv7_chunk_train<f16_t>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa,
-                                               (hipStream_t)stream);
+            e = launch_wkv7_chunk_train<f16_t>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa, ws,
+                                               ws_floats, (hipStream_t)stream);
         else
-            e = launch_wkv7_chunk_train<bf16_t>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa,
-                                                (hipStream_t)stream);
+            e = launch_wkv7_chunk_train<bf16_t>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa, ws,
+                                                ws_floats, (hipStream_t)stream);
         return launch_status(e, "wkv7_chunk2_kernel (training)");
     }
     RWKV7_DISPATCH(dtype, (launch_wkv7_train_fwd<IO>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt,

@@ -25,6 +25,7 @@
 // row).  A chunk whose per-token log-decay drops below kLogDecayFloor runs the
 // exact token-serial update instead, so every input gives the recurrence's result.
 #include "common.hpp"
+#include "wkv7_seg.hpp"
 
 #include <type_traits>
 
@@ -569,12 +570,18 @@ __device__ __forceinline__ void split1(float x, uint16_t& hi, uint16_t& lo) {
 // kernel also writes every token's sa_t = S_{t-1} a_t (float32, [tokens][H][64])
 // and the state after every 16th token of a sequence and after its last one
 // (ckpt [B][H][ceil(T/16)][64][64]), the layout the training backward reads.
-template <typename IO, bool TRAIN = false>
+//
+// segs.cps > 0: the sequences are walked in segments (wkv7_seg.hpp), block group g taking segment g.  CARRY is
+// the pass before the scan: only the state is walked, blockIdx.y = 0 from the identity without values (M),
+// 1 from zero, or from the sequence's initial state in its first segment (N); the first segment's M place
+// keeps a copy of that initial state, since the last segment's block of the full pass writes the final state
+// where the first one's may still have to be read.
+template <typename IO, bool TRAIN = false, bool CARRY = false>
 __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) void wkv7_chunk2_kernel(
     int H, int T_uniform, const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slot_idx, int pool_slots,
-    int total_tokens, float* __restrict__ state, const IO* __restrict__ r, const IO* __restrict__ w,
+    int total_tokens, WkvSegs segs, float* seg_m, float* seg_n, float* state, const IO* __restrict__ r, const IO* __restrict__ w,
     const IO* __restrict__ k, const IO* __restrict__ v, const IO* __restrict__ a, const IO* __restrict__ b,
-    IO* __restrict__ y, const float* __restrict__ s_init, float* __restrict__ ckpt, float* __restrict__ sa_out)
+    IO* __restrict__ y, const float* s_init, float* __restrict__ ckpt, float* __restrict__ sa_out)
 {
     typedef io_traits<IO> tr;
     // bf16 inputs are exact as bf16 MFMA operands: V (unscaled) has no lo plane, and
@@ -596,7 +603,12 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
     // batches keep their order (the ranking would cost more than the tail it
     // shortens).
     int s = unit / H;
-    if (cu_seqlens != nullptr) {
+    int seg = 0, nsg = 1;  // segment of the sequence
+    const bool ident = CARRY && blockIdx.y == 0;
+    if (segs.cps > 0) {
+        if (!wkvseg::locate(segs, unit / H, s, seg, nsg)) return;
+        if (CARRY && (seg == nsg - 1 || (ident && seg == 0))) return;
+    } else if (cu_seqlens != nullptr) {
         const int nseq = (int)(gridDim.x / (unsigned)H);
         if (nseq <= 256) {
             int* lens = sm.u.lens;
@@ -648,13 +660,19 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             }
         }
     };
-    if constexpr (TRAIN) {
-        if (s_init != nullptr)
-            tile_io(const_cast<float*>(s_init) + ((size_t)s * H + h) * (NH * NH), NH, false);
-        else
-            tile = f32x16{0.f};
-    } else {
-        tile_io(gS, NH, false);
+    // the initial state of the sequence: the pool slot's, or (training) s_init
+    const float* gInit = s_init != nullptr ? s_init + ((size_t)s * H + h) * (NH * NH) : TRAIN ? nullptr : gS;
+    if (seg > 0 || (nsg > 1 && !CARRY))  // found by the passes before (unused in CARRY)
+        gInit = seg > 0 ? seg_n + (size_t)(unit - H) * (NH * NH) : seg_m + (size_t)unit * (NH * NH);
+    if (gInit == nullptr || (CARRY && seg > 0))
+        tile = f32x16{0.f};
+    else
+        tile_io(const_cast<float*>(gInit), NH, false);
+    if (CARRY && seg == 0) tile_io(seg_m + (size_t)unit * (NH * NH), NH, true);
+    if (ident) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            tile[q] = 32 * ir_t + (lane & 31) == 32 * jt_t + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3) ? 1.f : 0.f;
     }
     store_state_planes(&sm.Sp[0][0][0], ir_t, jt_t, tile, lane);
     // a 64 x 64 state in the tiles' layout, one 16-byte store per group
@@ -679,7 +697,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         const size_t base = (size_t)t0c * C + h * NH;
         const IO* src[6] = {r, w, k, v, a, b};
 #pragma unroll
-        for (int q = 0; q < 6; ++q) {
+        for (int q = CARRY ? 1 : 0; q < 6; ++q) {  // (r is for y only)
             const __amdgpu_buffer_rsrc_t rs =
                 __builtin_amdgcn_make_buffer_rsrc(const_cast<IO*>(src[q] + base), 0, (int)bytes, 0x00020000);
 #pragma unroll
@@ -689,10 +707,13 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 raw[q][e] = make_uint2((uint32_t)u[0], (uint32_t)u[1]);
             }
         }
+        if (ident) raw[3][0] = raw[3][1] = make_uint2(0, 0);
     };
-    fetch(tb);
+    // the tokens this block walks
+    const int t_lo = tb + seg * segs.cps * L, t_hi = nsg > 1 ? min(te, t_lo + segs.cps * L) : te;
+    fetch(t_lo);
 
-    for (int t0 = tb; t0 < te; t0 += L) {
+    for (int t0 = t_lo; t0 < t_hi; t0 += L) {
         const int n = min(L, te - t0);
         [[maybe_unused]] const int ci = (t0 - tb) / L;  // chunk of the sequence: checkpoints 2 ci, 2 ci + 1
         // ---- A1: log2-decays of the thread's two tokens, their prefix over the chunk
@@ -748,7 +769,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 for (int e = 0; e < 2; ++e) {
                     const int t = 2 * tp + e;
                     const f32x4 ld = e == 0 ? ld_first : ld_first + lw[1];
-                    const f32x4 rv = unpack4<IO>(raw[0][e]), kv = unpack4<IO>(raw[2][e]);
+                    const f32x4 rv = CARRY ? f32x4{} : unpack4<IO>(raw[0][e]), kv = unpack4<IO>(raw[2][e]);
                     const f32x4 av = unpack4<IO>(raw[4][e]), bv = unpack4<IO>(raw[5][e]);
                     vv[e] = unpack4<IO>(raw[3][e]);
                     f32x4 rt, at, kh, bh;
@@ -763,9 +784,11 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                         bh[c] = bv[c] * iD;
                     }
                     uint2 hi, lo;
-                    split4(rt.x, rt.y, rt.z, rt.w, hi, lo);
-                    *reinterpret_cast<uint2*>(&sm.u.pa.Rt[0][t][j0]) = hi;
-                    *reinterpret_cast<uint2*>(&sm.u.pa.Rt[1][t][j0]) = lo;
+                    if constexpr (!CARRY) {
+                        split4(rt.x, rt.y, rt.z, rt.w, hi, lo);
+                        *reinterpret_cast<uint2*>(&sm.u.pa.Rt[0][t][j0]) = hi;
+                        *reinterpret_cast<uint2*>(&sm.u.pa.Rt[1][t][j0]) = lo;
+                    }
                     split4(at.x, at.y, at.z, at.w, hi, lo);
                     *reinterpret_cast<uint2*>(&sm.u.pa.At[0][t][j0]) = hi;
                     *reinterpret_cast<uint2*>(&sm.u.pa.At[1][t][j0]) = lo;
@@ -819,7 +842,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 for (int c = 0; c < 16; ++c) sa += tr::to_f32(a[off + q * 16 + c]) * sm.u.Sf[i][q * 16 + c];
                 sa += __shfl_xor(sa, 1, 64);
                 sa += __shfl_xor(sa, 2, 64);
-                const float vi = tr::to_f32(v[off + i]);
+                const float vi = ident ? 0.f : tr::to_f32(v[off + i]);
                 float yi = 0.f;
 #pragma unroll
                 for (int c = 0; c < 16; ++c) {
@@ -827,11 +850,13 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                     const float wd = expf(-expf(tr::to_f32(w[off + jj])));
                     const float sv = sm.u.Sf[i][jj] * wd + tr::to_f32(k[off + jj]) * vi + sa * tr::to_f32(b[off + jj]);
                     sm.u.Sf[i][jj] = sv;
-                    yi += sv * tr::to_f32(r[off + jj]);
+                    if constexpr (!CARRY) yi += sv * tr::to_f32(r[off + jj]);
                 }
-                yi += __shfl_xor(yi, 1, 64);
-                yi += __shfl_xor(yi, 2, 64);
-                if (q == 0) y[off + i] = tr::from_f32(yi);
+                if constexpr (!CARRY) {
+                    yi += __shfl_xor(yi, 1, 64);
+                    yi += __shfl_xor(yi, 2, 64);
+                    if (q == 0) y[off + i] = tr::from_f32(yi);
+                }
                 if constexpr (TRAIN) {
                     if (q == 0) sa_out[off + i] = sa;
                     if (t == 15 || t == n - 1) {  // checkpoint 2 ci (after token 15) or 2 ci + 1
@@ -845,14 +870,14 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             // back to the registers, and the hi/lo planes
             tile_io(&sm.u.Sf[0][0], SP, false);
             store_state_planes(&sm.Sp[0][0][0], ir_t, jt_t, tile, lane);
-            if (t0 + L < te) fetch(t0 + L);
+            if (t0 + L < t_hi) fetch(t0 + L);
             // the next chunk writes the region that holds Sf after its first barrier
             continue;
         }
 
         // the raw registers are free from here to the next phase A: fetch the next chunk (LDS barriers do not
         // wait for global loads, so these stay in flight through phases B to D)
-        if (t0 + L < te) fetch(t0 + L);
+        if (t0 + L < t_hi) fetch(t0 + L);
 
         // ---- B: two 32x32 tiles per wave, K = 64 over keys, sharing one operand:
         //   wave 0: X (value tile 0) and A_ab,   wave 1: X (value tile 1) and A_ak,
@@ -867,32 +892,46 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             const uint16_t* Q = wave < 2 ? &sm.u.pa.At[0][0][0] : &sm.u.pa.Rt[0][0][0];
             const uint16_t* P = (wave & 1) ? &sm.u.pa.Kh[0][0][0] : &sm.u.pa.Bh[0][0][0];
             f32x16 c1 = zero16;
-            for (int k0 = 0; k0 < NH; k0 += 16) {
-                const bf16x8_t s0 = fragSp(&sm.Sp[0][0][0], 32 * vt, k0, lane);
-                const bf16x8_t s1 = fragSp(&sm.Sp[1][0][0], 32 * vt, k0, lane);
-                const bf16x8_t q0 = frag(Q, KP, 0, k0, lane), q1 = frag(Q + RT_PLANE, KP, 0, k0, lane);
-                const bf16x8_t p0 = frag(P, KP, 0, k0, lane), p1 = frag(P + RT_PLANE, KP, 0, k0, lane);
-                accXY = mfma3(accXY, s0, s1, q0, q1);
-                c1 = mfma3(c1, p0, p1, q0, q1);
+            if constexpr (CARRY) {
+                // the state only: X on waves 0 / 1, A_ab and A_ak on waves 2 / 3
+                for (int k0 = 0; k0 < NH; k0 += 16) {
+                    const uint16_t* At = &sm.u.pa.At[0][0][0];
+                    const bf16x8_t q0 = frag(At, KP, 0, k0, lane), q1 = frag(At + RT_PLANE, KP, 0, k0, lane);
+                    if (wave < 2)
+                        accXY = mfma3(accXY, fragSp(&sm.Sp[0][0][0], 32 * vt, k0, lane),
+                                      fragSp(&sm.Sp[1][0][0], 32 * vt, k0, lane), q0, q1);
+                    else
+                        c1 = mfma3(c1, frag(P, KP, 0, k0, lane), frag(P + RT_PLANE, KP, 0, k0, lane), q0, q1);
+                }
+            } else {
+                for (int k0 = 0; k0 < NH; k0 += 16) {
+                    const bf16x8_t s0 = fragSp(&sm.Sp[0][0][0], 32 * vt, k0, lane);
+                    const bf16x8_t s1 = fragSp(&sm.Sp[1][0][0], 32 * vt, k0, lane);
+                    const bf16x8_t q0 = frag(Q, KP, 0, k0, lane), q1 = frag(Q + RT_PLANE, KP, 0, k0, lane);
+                    const bf16x8_t p0 = frag(P, KP, 0, k0, lane), p1 = frag(P + RT_PLANE, KP, 0, k0, lane);
+                    accXY = mfma3(accXY, s0, s1, q0, q1);
+                    c1 = mfma3(c1, p0, p1, q0, q1);
+                }
             }
+            constexpr int kA = CARRY ? 2 : 0;  // the wave with A_ab; the next one has A_ak
             // lane holds [s = 8g + 4(l/32) + e][t = l%32]
             const int tcol = lane & 31;
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 const int srow = 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-                const bool keep = wave < 2 ? srow < tcol : srow <= tcol;
+                const bool keep = CARRY || wave < 2 ? srow < tcol : srow <= tcol;
                 c1[q] = keep ? c1[q] : 0.f;
             }
             // the products overwrite the planes they were computed from
             lds_barrier();
-            if (wave == 0) {
+            if (wave == kA) {
                 float* AT = &sm.u.pb.AT[0][0];
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
                     *reinterpret_cast<f32x4*>(AT + tcol * TP + 8 * g + 4 * (lane >> 5)) =
                         f32x4{c1[4 * g], c1[4 * g + 1], c1[4 * g + 2], c1[4 * g + 3]};
-            } else {
-                uint16_t* out = wave == 1 ? &sm.u.pb.AakT[0][0][0] : wave == 2 ? &sm.u.pb.BrbT[0][0][0]
+            } else if (!CARRY || wave == kA + 1) {
+                uint16_t* out = wave == kA + 1 ? &sm.u.pb.AakT[0][0][0] : wave == 2 ? &sm.u.pb.BrbT[0][0][0]
                                                                                : &sm.u.pb.BrkT[0][0][0];
                 store_planes_T(out, TQ, T32_PLANE, 0, 0, c1, lane);
             }
@@ -900,7 +939,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         lds_barrier();
 
         // ---- C: X += V^T A_ak (waves 0/1), stored as X^T; Y += V^T B_rk (waves 2/3) --
-        {
+        if (!CARRY || wave < 2) {
             const uint16_t* M = wave < 2 ? &sm.u.pb.AakT[0][0][0] : &sm.u.pb.BrkT[0][0][0];
             for (int k0 = 0; k0 < L; k0 += 16) {
                 const bf16x8_t a0 = frag(M, TQ, 0, k0, lane), a1 = frag(M + T32_PLANE, TQ, 0, k0, lane);
@@ -1032,7 +1071,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             if (n > 16) put_state(gCk + (size_t)(2 * ci + 1) * (NH * NH), tile);  // after the chunk's last token
         }
         store_state_planes(&sm.Sp[0][0][0], ir_t, jt_t, tile, lane);
-        if (wave >= 2) {
+        if (!CARRY && wave >= 2) {
             for (int k0 = 0; k0 < L; k0 += 16) {
                 const bf16x8_t p0 = frag(&sm.u.pb.BrbT[0][0][0], TQ, 0, k0, lane);
                 const bf16x8_t p1 = frag(&sm.u.pb.BrbT[1][0][0], TQ, 0, k0, lane);
@@ -1054,27 +1093,101 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         // reads the state planes written here after two of them).
     }
     // the final state, straight from the registers
-    if (gS != nullptr) tile_io(gS, NH, true);
+    if constexpr (CARRY) {
+        tile_io((ident ? seg_m : seg_n) + (size_t)unit * (NH * NH), NH, true);
+    } else {
+        if (gS != nullptr && seg == nsg - 1) tile_io(gS, NH, true);
+    }
+}
+
+// Cost of a launch per chunk of its walk, in microseconds: a block alone on its CU takes 4.55 us per chunk
+// (bf16, H = 32), two on a CU 6.2 us for both (float16 has one block per CU); more blocks run in rounds.
+float walk_cost(int64_t blocks, bool two_per_cu)
+{
+    if (blocks <= 256) return 4.55f;
+    return two_per_cu ? 6.2f * (float)((blocks + 511) / 512) : 4.55f * (float)((blocks + 255) / 256);
 }
 
 }  // namespace
 
+// Segments of a launch; cps = 0 (unsplit) where that is not slower.  n segments per sequence cost the state
+// pass (0.75 of a full walk per chunk; 2 n - 3 blocks per unit), the scan (0.5 us a step) and the full pass
+// over n segments, against one block per unit over the whole sequence.  Ragged sequences count with their
+// average length.  Measured (us, bf16, unsplit -> split): 12 units 128 tokens 22 -> 20, 12 x 512 76 -> 31,
+// 32 x 1000 148 -> 54, 32 x 4096 580 -> 150, 64 x 256 40 -> 35, 64 x 2048 291 -> 146, 128 x 1000 148 -> 131;
+// not split by the model and slower split: 32 x 64 13 -> 18, 64 x 160 27 -> 30, 128 x 384 58 -> 60,
+// 192 x 4096 583 -> 679, 256 x 4096 588 -> 744.
+static WkvSegs plan_segments(int nseq, int H, int T_uniform, const int32_t* cu, int total, bool two_per_cu)
+{
+    WkvSegs m = {nseq, 0, 0, T_uniform, total, cu};
+    const int64_t units = (int64_t)nseq * H;
+    const int per_seq = cu == nullptr ? (T_uniform + L - 1) / L : (int)(((int64_t)total + nseq * L - 1) / ((int64_t)nseq * L));
+    if (units >= 256) return m;
+    float best = per_seq * walk_cost(units, two_per_cu);
+    for (int n = 2; n <= 32 && n <= per_seq; ++n) {
+        const int cps = (per_seq + n - 1) / n, nn = (per_seq + cps - 1) / cps;
+        const float cost = cps * (0.75f * walk_cost(units * (2 * nn - 3), two_per_cu) +
+                                  walk_cost(units * nn, two_per_cu)) + 0.5f * nn + 9.f;
+        if (cost < best) {
+            best = cost;
+            m.cps = cps;
+        }
+    }
+    if (m.cps > 0)
+        m.gmax = cu == nullptr ? nseq * ((per_seq + m.cps - 1) / m.cps) : total / (m.cps * L) + nseq;
+    return m;
+}
+
+// floats of workspace with which a 16-bit launch of these sizes may run in segments (cu: any non-null
+// pointer for ragged sequences); without it, it runs unsplit
+int64_t wkv7_chunk_ws(int nseq, int H, int T_uniform, bool ragged, int total, bool two_per_cu)
+{
+    static const int32_t some = 0;
+    const WkvSegs m = plan_segments(nseq, H, T_uniform, ragged ? &some : nullptr, total, two_per_cu);
+    return (int64_t)m.gmax * H * 2 * NH * NH;
+}
+
+template <typename IO, bool TRAIN>
+static hipError_t launch_chunk2(int nseq, int H, int T_uniform, const int32_t* cu_seqlens, const int32_t* slot_idx,
+                                int pool_slots, int total, float* state, const void* r, const void* w, const void* k,
+                                const void* v, const void* a, const void* b, void* y, const float* s0, float* ckpt,
+                                float* sa, float* ws, int64_t ws_floats, hipStream_t stream)
+{
+    WkvSegs m = plan_segments(nseq, H, T_uniform, cu_seqlens, total, std::is_same<IO, bf16_t>::value);
+    const int64_t half = (int64_t)m.gmax * H * NH * NH;
+    if (m.cps > 0 && (ws == nullptr || ws_floats < 2 * half)) m.cps = 0;
+    float *sm = ws, *sn = ws + half;
+    const unsigned groups = m.cps > 0 ? (unsigned)m.gmax : (unsigned)nseq;
+    if (m.cps > 0) {
+        hipLaunchKernelGGL((wkv7_chunk2_kernel<IO, false, true>), dim3(groups * (unsigned)H, 2), dim3(256), 0, stream,
+                           H, T_uniform, cu_seqlens, slot_idx, pool_slots, total, m, sm, sn, TRAIN ? nullptr : state,
+                           (const IO*)r, (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a, (const IO*)b,
+                           (IO*)y, s0, nullptr, nullptr);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = launch_wkv7_scan_forward(m, H, sm, sn, stream);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((wkv7_chunk2_kernel<IO, TRAIN, false>), dim3(groups * (unsigned)H), dim3(256), 0, stream, H,
+                       T_uniform, cu_seqlens, slot_idx, pool_slots, total, m, sm, sn, state, (const IO*)r,
+                       (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a, (const IO*)b, (IO*)y, s0, ckpt, sa);
+    return hipGetLastError();
+}
+
 template <typename IO>
 hipError_t launch_wkv7_chunk(int nseq, int H, int T_uniform, const int32_t* cu_seqlens, const int32_t* slot_idx,
                              int pool_slots, int total_tokens, float* state, const void* r, const void* w,
-                             const void* k, const void* v, const void* a, const void* b, void* y, hipStream_t stream)
+                             const void* k, const void* v, const void* a, const void* b, void* y, float* ws,
+                             int64_t ws_floats, hipStream_t stream)
 {
     if constexpr (sizeof(IO) == 4) {
         hipLaunchKernelGGL(wkv7_chunk_kernel<IO>, dim3((unsigned)nseq * (unsigned)H), dim3(256), 0, stream, H,
                            T_uniform, cu_seqlens, slot_idx, pool_slots, total_tokens, state, (const IO*)r,
                            (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a, (const IO*)b, (IO*)y);
+        return hipGetLastError();
     } else {
-        hipLaunchKernelGGL((wkv7_chunk2_kernel<IO, false>), dim3((unsigned)nseq * (unsigned)H), dim3(256), 0, stream,
-                           H, T_uniform, cu_seqlens, slot_idx, pool_slots, total_tokens, state, (const IO*)r,
-                           (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a, (const IO*)b, (IO*)y, nullptr,
-                           nullptr, nullptr);
+        return launch_chunk2<IO, false>(nseq, H, T_uniform, cu_seqlens, slot_idx, pool_slots, total_tokens, state, r,
+                                        w, k, v, a, b, y, nullptr, nullptr, nullptr, ws, ws_floats, stream);
     }
-    return hipGetLastError();
 }
 
 // The training operator's forward in chunked form (16-bit I/O): B sequences of T
@@ -1083,27 +1196,23 @@ hipError_t launch_wkv7_chunk(int nseq, int H, int T_uniform, const int32_t* cu_s
 template <typename IO>
 hipError_t launch_wkv7_chunk_train(int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
                                    const void* a, const void* b, void* y, const float* s0, float* s_out, float* ckpt,
-                                   float* sa, hipStream_t stream)
+                                   float* sa, float* ws, int64_t ws_floats, hipStream_t stream)
 {
     static_assert(sizeof(IO) == 2, "16-bit inputs");
-    hipLaunchKernelGGL((wkv7_chunk2_kernel<IO, true>), dim3((unsigned)B * (unsigned)H), dim3(256), 0, stream, H, T,
-                       nullptr, nullptr, B, B * T, s_out, (const IO*)r, (const IO*)w, (const IO*)k, (const IO*)v,
-                       (const IO*)a, (const IO*)b, (IO*)y, s0, ckpt, sa);
-    return hipGetLastError();
+    return launch_chunk2<IO, true>(B, H, T, nullptr, nullptr, B, B * T, s_out, r, w, k, v, a, b, y, s0, ckpt, sa, ws,
+                                   ws_floats, stream);
 }
 
-template hipError_t launch_wkv7_chunk<float>(int, int, int, const int32_t*, const int32_t*, int, int, float*, const void*,
-                                             const void*, const void*, const void*, const void*, const void*, void*,
-                                             hipStream_t);
-template hipError_t launch_wkv7_chunk<bf16_t>(int, int, int, const int32_t*, const int32_t*, int, int, float*,
-                                              const void*, const void*, const void*, const void*, const void*,
-                                              const void*, void*, hipStream_t);
-template hipError_t launch_wkv7_chunk<f16_t>(int, int, int, const int32_t*, const int32_t*, int, int, float*, const void*,
-                                             const void*, const void*, const void*, const void*, const void*, void*,
-                                             hipStream_t);
-template hipError_t launch_wkv7_chunk_train<bf16_t>(int, int, int, const void*, const void*, const void*, const void*,
-                                                    const void*, const void*, void*, const float*, float*, float*,
-                                                    float*, hipStream_t);
-template hipError_t launch_wkv7_chunk_train<f16_t>(int, int, int, const void*, const void*, const void*, const void*,
-                                                   const void*, const void*, void*, const float*, float*, float*,
-                                                   float*, hipStream_t);
+#define RWKV7_INST(IO)                                                                                               \
+    template hipError_t launch_wkv7_chunk<IO>(int, int, int, const int32_t*, const int32_t*, int, int, float*,       \
+                                              const void*, const void*, const void*, const void*, const void*,      \
+                                              const void*, void*, float*, int64_t, hipStream_t);
+#define RWKV7_INST_TRAIN(IO)                                                                                         \
+    template hipError_t launch_wkv7_chunk_train<IO>(int, int, int, const void*, const void*, const void*,            \
+                                                    const void*, const void*, const void*, void*, const float*,     \
+                                                    float*, float*, float*, float*, int64_t, hipStream_t);
+RWKV7_INST(float)
+RWKV7_INST(bf16_t)
+RWKV7_INST(f16_t)
+RWKV7_INST_TRAIN(bf16_t)
+RWKV7_INST_TRAIN(f16_t)

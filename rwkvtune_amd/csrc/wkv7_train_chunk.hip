@@ -39,6 +39,7 @@
 // with no bank conflicts; the matrix cores are busy 13%.  Four waves per SIMD with packed
 // operands took 1.23 ms where two waves per SIMD that split operands at each read took 1.5.
 #include "wkv7_mm.hpp"
+#include "wkv7_seg.hpp"
 
 #include <type_traits>
 
@@ -624,64 +625,6 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
     }
 }
 
-// G at every segment start, last to first: G_s = G_{s+1} Q_s + H_s, written over H.  Rows of G are
-// independent: a block takes 16 of them (wave w: columns 16 w ..), v_mfma_f32_16x16x4_f32 throughout.
-// The chain's step is a few hundred cycles against a memory latency of a microsecond or two, so Q and H
-// are loaded kAhead segments ahead.
-constexpr int kAhead = 4;
-__global__ __launch_bounds__(256) void wkv7_train_bwd_scan_kernel(int nseg, const float* __restrict__ seg_q,
-                                                                  float* __restrict__ seg_h)
-{
-    __shared__ __attribute__((aligned(16))) float g[2][16][SP];
-    const int unit = blockIdx.x >> 2, i0 = 16 * (blockIdx.x & 3);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = lane & 15, h = lane >> 4;
-    const size_t base = (size_t)unit * nseg * (NH * NH);
-    const int er = tid >> 4, ec = 4 * (tid & 15);
-    float q[kAhead][16], hh[kAhead][4];
-    auto load = [&](int s, float (&qq)[16], float (&h4)[4]) {
-        const float* Q = seg_q + base + (size_t)s * (NH * NH) + 4 * h * NH + 16 * wave + c;
-        const float* Hs = seg_h + base + (size_t)s * (NH * NH) + (i0 + 4 * h) * NH + 16 * wave + c;
-#pragma unroll
-        for (int m = 0; m < 16; ++m) qq[m] = Q[(16 * (m >> 2) + (m & 3)) * NH];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h4[e] = Hs[e * NH];
-    };
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u)
-        if (nseg - 2 - u >= 1) load(nseg - 2 - u, q[u], hh[u]);
-    // the last segment's H is already its G_start
-    *reinterpret_cast<f32x4*>(&g[0][er][ec]) =
-        *reinterpret_cast<const f32x4*>(seg_h + base + (size_t)(nseg - 1) * (NH * NH) + (i0 + er) * NH + ec);
-    __syncthreads();
-    for (int s0 = nseg - 2; s0 >= 1; s0 -= kAhead) {
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const int s = s0 - u;
-            if (s < 1) break;  // uniform
-            f32x4 acc0 = {hh[u][0], hh[u][1], hh[u][2], hh[u][3]}, acc1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int m4 = 0; m4 < 4; ++m4) {
-                const f32x4 x = *reinterpret_cast<const f32x4*>(&g[u & 1][c][16 * m4 + 4 * h]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (m4 & 1) acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], q[u][4 * m4 + e], acc1, 0, 0, 0);
-                    else acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], q[u][4 * m4 + e], acc0, 0, 0, 0);
-                }
-            }
-            if (s - kAhead >= 1) load(s - kAhead, q[u], hh[u]);
-            float* Hs = seg_h + base + (size_t)s * (NH * NH) + (i0 + 4 * h) * NH + 16 * wave + c;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float x = acc0[e] + acc1[e];
-                g[(u & 1) ^ 1][4 * h + e][16 * wave + c] = x;
-                Hs[e * NH] = x;
-            }
-            __syncthreads();
-        }
-    }
-}
-
 // Segments per unit: enough blocks for the 256 CUs (one block each), none shorter than a chunk.
 int bwd_segments(int64_t units, int T, int* cps) {
     const int nchunk = (T + L - 1) / L;
@@ -729,8 +672,7 @@ hipError_t launch_wkv7_train_bwd_chunk(int B, int T, int H, const void* r, const
                              : launch(wkv7_train_bwd_chunk_kernel<IO, false, false>, two, kBwdThreads<false>, sizeof(BwdLds<false>));
         if (e != hipSuccess) return e;
         if (nseg > 2) {
-            hipLaunchKernelGGL(wkv7_train_bwd_scan_kernel, dim3((unsigned)(4 * units)), dim3(256), 0, st, nseg, q, h);
-            e = hipGetLastError();
+            e = launch_wkv7_scan_backward(units, nseg, q, h, st);
             if (e != hipSuccess) return e;
         }
     }

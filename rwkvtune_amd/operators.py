@@ -79,6 +79,13 @@ def _contig(*ts):
     return out
 
 
+def _segment_ws(dtype, nseq, H, T, total, ragged, device):
+    """``(workspace tensor or None, floats)`` with which a chunked call of few
+    (sequence, head) pairs walks its sequences in segments side by side."""
+    n = _lib.load().rwkv7_wkv_segment_ws_floats(_lib.dtype_code(dtype), nseq, H, T, total, int(ragged))
+    return (torch.empty(n, dtype=torch.float32, device=device), n) if n > 0 else (None, 0)
+
+
 def _check_out(y, r):
     if y.shape != r.shape or y.dtype != r.dtype or y.device != r.device or not y.is_contiguous():
         raise RuntimeError("y must be a contiguous tensor with r's shape, dtype and device")
@@ -104,8 +111,9 @@ def wkv7s_forward(state, r, w, k, v, a, b, head_size: int = HEAD_SIZE):
         raise RuntimeError(f"state must be a contiguous [B={B}, H={H}, {head_size}, {head_size}] tensor")
     r, w, k, v, a, b = _contig(r, w, k, v, a, b)
     y = torch.empty(r.shape, dtype=r.dtype, device=r.device)
-    _lib.call("rwkv7s_forward", _lib.dtype_code(r.dtype), B, T, C, H, _lib.ptr(state),
-              *(_lib.ptr(t) for t in (r, w, k, v, a, b)), _lib.ptr(y), _lib.stream_of(r))
+    ws, n = _segment_ws(r.dtype, B, H, T, B * T, False, r.device)
+    _lib.call("rwkv7s_forward_ws", _lib.dtype_code(r.dtype), B, T, C, H, _lib.ptr(state),
+              *(_lib.ptr(t) for t in (r, w, k, v, a, b)), _lib.ptr(y), _lib.ptr(ws), n, _lib.stream_of(r))
     return y
 
 
@@ -154,8 +162,9 @@ def _train_forward(w, q, k, v, a, b, s0=None, s_out=None):
     ckpt = torch.empty((B, H, nck, N, N), dtype=torch.float32, device=dev)
     sa = torch.empty((B, T, H, N), dtype=torch.float32, device=dev)
     P = _lib.ptr
-    _lib.call("rwkv7_wkv_train_forward", _lib.dtype_code(q.dtype), B, T, H, P(q), P(w), P(k), P(v), P(a), P(b),
-              P(y), P(s0), P(s_out), P(ckpt), P(sa), _lib.stream_of(q))
+    ws, n = _segment_ws(q.dtype, B, H, T, B * T, False, dev)
+    _lib.call("rwkv7_wkv_train_forward_ws", _lib.dtype_code(q.dtype), B, T, H, P(q), P(w), P(k), P(v), P(a), P(b),
+              P(y), P(s0), P(s_out), P(ckpt), P(sa), P(ws), n, _lib.stream_of(q))
     return y, ckpt, sa
 
 
@@ -390,7 +399,8 @@ def wkv7_prefill(state_pool, slot_idx, cu_seqlens, r, w, k, v, a, b, y=None, chu
         y = torch.empty(r.shape, dtype=r.dtype, device=r.device)
     _check_out(y, r)
     ins = _contig(r, w, k, v, a, b)  # kept alive until the launch is enqueued
-    _lib.call("rwkv7_wkv_prefill", _lib.dtype_code(r.dtype), nseq, H, total,
+    ws, n = _segment_ws(r.dtype, nseq, H, 0, total, True, r.device)
+    _lib.call("rwkv7_wkv_prefill_ws", _lib.dtype_code(r.dtype), nseq, H, total,
               _lib.ptr(cu_seqlens), _lib.ptr(slot_idx), _lib.ptr(state_pool), S,
-              *(_lib.ptr(t) for t in ins), _lib.ptr(y), int(chunk_len), _lib.stream_of(r))
+              *(_lib.ptr(t) for t in ins), _lib.ptr(y), int(chunk_len), _lib.ptr(ws), n, _lib.stream_of(r))
     return y
