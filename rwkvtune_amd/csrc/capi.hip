@@ -74,6 +74,8 @@ int chunk_dispatch(int dtype, int nseq, int H, int T_uniform, const int32_t* cu,
                    int total, float* state, const void* r, const void* w, const void* k, const void* v,
                    const void* a, const void* b, void* y, float* ws, int64_t ws_floats, hipStream_t st) {
     hipError_t e;
+    if (dtype == RWKV7_DTYPE_F32 && H > (1 << 17))  // rows too long for 32-bit offsets within a chunk
+        return seq_dispatch(dtype, nseq, H, T_uniform, cu, slot, pool_slots, total, state, r, w, k, v, a, b, y, st);
     switch (dtype) {
         case RWKV7_DTYPE_F32:
             e = launch_wkv7_chunk<float>(nseq, H, T_uniform, cu, slot, pool_slots, total, state, r, w, k, v, a, b, y,
@@ -116,7 +118,7 @@ extern "C" const char* rwkv7_last_error(void) { return g_err; }
 extern "C" int64_t rwkv7_wkv_segment_ws_floats(int dtype, int64_t nseq, int64_t H, int64_t T, int64_t total_tokens,
                                                int ragged) {
     ok();
-    if (!dtype_ok(dtype) || dtype == RWKV7_DTYPE_F32 || nseq <= 0 || H <= 0 || total_tokens <= 0 ||
+    if (!dtype_ok(dtype) || nseq <= 0 || H <= 0 || total_tokens <= 0 ||
         (ragged == 0 && T <= 0) || nseq * H > kMaxInt || T > kMaxInt || total_tokens > kMaxInt)
         return 0;  // sizes that the call itself refuses or that have nothing to split
     return wkv7_chunk_ws((int)nseq, (int)H, ragged ? 0 : (int)T, ragged != 0, (int)total_tokens,
@@ -625,16 +627,12 @@ extern "C" int rwkv7_wkv_train_forward_ws(int dtype, int64_t B, int64_t T, int64
     if (f32_misaligned(ckpt) || f32_misaligned(s0) || f32_misaligned(s_out) || f32_misaligned(ws))
         return fail(RWKV7_ERR_INVALID, "rwkv7_wkv_train_forward: checkpoints and states must be 16-byte aligned");
     hipError_t e;
-    // 16-bit inputs aligned to 4 elements run the chunked kernel (32-token matrix
-    // form on the matrix cores); float32 inputs keep the token-serial kernel
-    if (dtype != RWKV7_DTYPE_F32 && B * T <= kMaxInt && !misaligned(dtype, nullptr, r, w, k, v, a, b)) {
-        if (dtype == RWKV7_DTYPE_F16)
-            e = launch_wkv7_chunk_train<f16_t>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa, ws,
-                                               ws_floats, (hipStream_t)stream);
-        else
-            e = launch_wkv7_chunk_train<bf16_t>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt, sa, ws,
-                                                ws_floats, (hipStream_t)stream);
-        return launch_status(e, "wkv7_chunk2_kernel (training)");
+    // inputs aligned to 4 elements run in 32-token chunks on the matrix cores, others token by token
+    if (B * T <= kMaxInt && H <= (1 << 17) && !misaligned(dtype, nullptr, r, w, k, v, a, b) &&
+        !(dtype == RWKV7_DTYPE_F32 && (f32_misaligned((const float*)y) || f32_misaligned(sa)))) {
+        RWKV7_DISPATCH(dtype, (launch_wkv7_chunk_train<IO>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out,
+                                                           ckpt, sa, ws, ws_floats, (hipStream_t)stream)));
+        return launch_status(e, "chunked WKV7 training forward");
     }
     RWKV7_DISPATCH(dtype, (launch_wkv7_train_fwd<IO>((int)B, (int)T, (int)H, r, w, k, v, a, b, y, s0, s_out, ckpt,
                                                      sa, (hipStream_t)stream)));

@@ -61,13 +61,14 @@ __device__ __forceinline__ float sum8(float x) {
     return x + dpp_xor7(x);
 }
 
-template <bool GRADS>
+// DT: type of the log2-decay sums (double for float32 inputs)
+template <bool GRADS, typename DT>
 struct __attribute__((aligned(16))) BwdLds {
     float Rt[L][SP], At[L][SP], Bh[L][SP];  // scaled operands [t][j]
     float DY[L][SP], X[L][SP];              // [t][i]
     float G[NH][SP];                        // G^ of the chunk [i][j]
     float T[L][TP], AbT[L][TP], Rb[L][TP];  // T [s][t], A_ab^T [t][s], B_rb [s][t]
-    float tot[16][NH];
+    DT tot[GRADS ? 16 : 8][NH];
     int slow[16];
     struct Grads {
         float Z[L][SP], Kh[L][SP], V[L][SP], SA[L][SP], S[NH][SP];
@@ -77,8 +78,8 @@ struct __attribute__((aligned(16))) BwdLds {
     struct None {};
     typename std::conditional<GRADS, Grads, None>::type g;
 };
-static_assert(sizeof(BwdLds<true>) <= 160 * 1024, "one block per CU");
-static_assert(sizeof(BwdLds<false>) <= 80 * 1024, "two blocks per CU");
+static_assert(sizeof(BwdLds<true, double>) <= 160 * 1024, "one block per CU");
+static_assert(sizeof(BwdLds<false, double>) <= 80 * 1024, "two blocks per CU");
 
 template <bool GRADS>
 constexpr int kBwdThreads = GRADS ? 1024 : 512;
@@ -106,7 +107,8 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
     constexpr int CH = NH * L / kBwdThreads<GRADS>;       // channels per thread of the element-wise phases
     constexpr int TPW = L / NW;                           // tokens per wave there
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    BwdLds<GRADS>& sm = *reinterpret_cast<BwdLds<GRADS>*>(smem);
+    typedef typename std::conditional<FI, double, float>::type DT;
+    BwdLds<GRADS, DT>& sm = *reinterpret_cast<BwdLds<GRADS, DT>*>(smem);
     const int tid = threadIdx.x, lane0 = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int unit = blockIdx.x / nseg;
@@ -207,26 +209,24 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
             qv.get(xv);
             qs.get(xsa);
         }
-        float lw2[CH], pre[CH];
+        DT lw2[CH], pre[CH];
         bool slow = false;
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
-            const float x = tk < n ? -(FI ? expf(xw[e]) : ex2(xw[e] * kLog2e)) * kLog2e : 0.f;
-            slow |= !(x >= kLog2DecayFloor);
+            const DT x = tk < n ? -(DT)(FI ? expf(xw[e]) : ex2(xw[e] * kLog2e)) * (DT)1.4426950408889634 : (DT)0;
+            slow |= !(x >= (DT)kLog2DecayFloor);
             lw2[e] = x;
             if constexpr (TPW == 4) {
-                const float p1 = lane_xor16(x), p2 = lane_xor32(x + p1);
-                pre[e] = (grp >= 2 ? p2 : 0.f) + ((grp & 1) ? p1 : 0.f);  // tokens of the wave before this one
+                const DT p1 = xor16(x), p2 = xor32(x + p1);
+                pre[e] = (grp >= 2 ? p2 : (DT)0) + ((grp & 1) ? p1 : (DT)0);  // tokens of the wave before this one
             } else {
-                const float p = lane_xor32(x);
-                pre[e] = grp ? p : 0.f;
+                const DT p = xor32(x);
+                pre[e] = grp ? p : (DT)0;
             }
         }
         if (grp == TPW - 1) {
-            float x[CH];
 #pragma unroll
-            for (int e = 0; e < CH; ++e) x[e] = pre[e] + lw2[e];
-            put_ch<false, CH>(&sm.tot[wave][j0], x);
+            for (int e = 0; e < CH; ++e) sm.tot[wave][j0 + e] = pre[e] + lw2[e];
         }
         const bool wave_slow = __ballot(slow) != 0;
         if (lane == 0) sm.slow[wave] = wave_slow ? 1 : 0;
@@ -352,21 +352,20 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
         }
 
         // ---- scaled operands -----------------------------------------------------------------------
-        float before[CH];  // log2 D before this token
+        DT before[CH];  // log2 D before this token
 #pragma unroll
         for (int e = 0; e < CH; ++e) before[e] = pre[e];
 #pragma unroll
         for (int q = 0; q < NW - 1; ++q) {
             if (q < wave) {  // uniform
-                float x[CH];
-                get_ch<CH>(&sm.tot[q][j0], x);
 #pragma unroll
-                for (int e = 0; e < CH; ++e) before[e] += x[e];
+                for (int e = 0; e < CH; ++e) before[e] += sm.tot[q][j0 + e];
             }
         }
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
-            const float ld = before[e] + lw2[e], iD = ex2(-ld);
+            const DT ld = before[e] + lw2[e];
+            const float iD = ex2(-ld);
             xr[e] *= ex2(ld);
             xa[e] *= ex2(before[e]);
             xb[e] *= iD;
@@ -411,12 +410,12 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
             for (int e = 0; e < CH; ++e) cj[e] += x[e];
         }
         if (wave < 4) {  // G^ = G diag(D_L)
-            float all = 0.f;
+            DT all = 0;
 #pragma unroll
             for (int q = 0; q < NW; ++q) all += sm.tot[q][gj + (lane & 31)];
-            all = ex2(all);
+            const float DL = ex2(all);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) G[q] *= all;
+            for (int q = 0; q < 16; ++q) G[q] *= DL;
             put<PG>(&sm.G[0][0], SP, gi, gj, G, lane);
         }
         if (c > c_lo) fetch(c - 1, id);
@@ -583,26 +582,28 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
                     suf[e] = x + (grp ? 0.f : p);
                 }
             }
-            if (grp == 0) put_ch<false, CH>(&sm.tot[wave][j0], suf);
+            if (grp == 0) {
+#pragma unroll
+                for (int e = 0; e < CH; ++e) sm.tot[wave][j0 + e] = suf[e];
+            }
             lds_barrier();
 #pragma unroll
             for (int q = 1; q < NW; ++q) {
                 if (q > wave) {  // uniform
-                    float x[CH];
-                    get_ch<CH>(&sm.tot[q][j0], x);
 #pragma unroll
-                    for (int e = 0; e < CH; ++e) suf[e] += x[e];
+                    for (int e = 0; e < CH; ++e) suf[e] += (float)sm.tot[q][j0 + e];
                 }
             }
             const uint32_t o = (uint32_t)tk * stride + j0 * sizeof(IO);
 #pragma unroll
             for (int e = 0; e < CH; ++e) {
-                const float ld = before[e] + lw2[e], iD = ex2(-ld);
+                const DT ld = before[e] + lw2[e];
+                const float iD = ex2(-ld);
                 gr[e] *= ex2(ld);
                 ga[e] *= ex2(before[e]);
                 gk[e] *= iD;
                 gb[e] *= iD;
-                suf[e] = (suf[e] + cj[e] - ya[e]) * (lw2[e] * 0.6931471805599453f);  // log-decay -exp(w)
+                suf[e] = (suf[e] + cj[e] - ya[e]) * (float)(lw2[e] * (DT)0.6931471805599453);  // log-decay -exp(w)
             }
             store_ch<IO, CH>(rows(dr, c), o, gr);
             store_ch<IO, CH>(rows(da, c), o, ga);
@@ -665,19 +666,20 @@ hipError_t launch_wkv7_train_bwd_chunk(int B, int T, int H, const void* r, const
                            q, h, (IO*)dr, (IO*)dw, (IO*)dk, (IO*)dv, (IO*)da, (IO*)db, ds0);
         return hipGetLastError();
     };
-    const bool exact = ds0 != nullptr || sizeof(IO) == 4;
     const dim3 full((unsigned)(units * nseg)), two((unsigned)(units * nseg), 2);
-    if (nseg > 1) {
-        hipError_t e = exact ? launch(wkv7_train_bwd_chunk_kernel<IO, false, true>, two, kBwdThreads<false>, sizeof(BwdLds<false>))
-                             : launch(wkv7_train_bwd_chunk_kernel<IO, false, false>, two, kBwdThreads<false>, sizeof(BwdLds<false>));
-        if (e != hipSuccess) return e;
-        if (nseg > 2) {
-            e = launch_wkv7_scan_backward(units, nseg, q, h, st);
+    typedef typename std::conditional<sizeof(IO) == 4, double, float>::type DT;
+    auto passes = [&](auto exact) -> hipError_t {
+        constexpr bool EX = decltype(exact)::value;
+        if (nseg > 1) {
+            hipError_t e = launch(wkv7_train_bwd_chunk_kernel<IO, false, EX>, two, kBwdThreads<false>,
+                                  sizeof(BwdLds<false, DT>));
+            if (e == hipSuccess && nseg > 2) e = launch_wkv7_scan_backward(units, nseg, q, h, st);
             if (e != hipSuccess) return e;
         }
-    }
-    return exact ? launch(wkv7_train_bwd_chunk_kernel<IO, true, true>, full, kBwdThreads<true>, sizeof(BwdLds<true>))
-                 : launch(wkv7_train_bwd_chunk_kernel<IO, true, false>, full, kBwdThreads<true>, sizeof(BwdLds<true>));
+        return launch(wkv7_train_bwd_chunk_kernel<IO, true, EX>, full, kBwdThreads<true>, sizeof(BwdLds<true, DT>));
+    };
+    if constexpr (sizeof(IO) == 4) return passes(std::true_type());
+    else return ds0 != nullptr ? passes(std::true_type()) : passes(std::false_type());
 }
 
 #define RWKV7_INST(IO)                                                                                              \

@@ -111,3 +111,29 @@ def test_workspace_too_small_runs_unsplit(gpu_device):
     _lib.call("rwkv7s_forward", *args, P(s2), *(P(x) for x in ins), P(y2), _lib.stream_of(y2))
     torch.cuda.synchronize()
     assert torch.equal(y1, y2) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("lens", [[1], [31, 32, 33], [64, 1, 200], [0, 600, 96], [1500]])
+@pytest.mark.parametrize("strong", [False, True])
+def test_float32_chunks(gpu_device, lens, strong):
+    """The float32 chunked kernel (float32 MFMAs; segmented from a few hundred tokens on) against the float64
+    recurrence: 64-term float32 sums carried over the sequence, 2e-6 of the largest magnitude."""
+    print(f"[case] float32 prefill lens={lens} strong={strong}", flush=True)
+    H, total, n = 4, sum(lens), len(lens)
+    ins = [x.to(gpu_device) for x in wkv_inputs((total,), H, seed=total, dtype=torch.float32).as_tuple()]
+    if strong:
+        ins[1][total // 2, 70] = 1.0
+        ins[1][total - 1, 3] = 0.5
+    cu = torch.tensor(cu_seqlens_of(lens), dtype=torch.int32, device=gpu_device)
+    pool0 = wkv_state(n, H).to(gpu_device)
+    pool = pool0.clone()
+    y = ops.wkv7_prefill(pool, None, cu, *ins)
+    torch.cuda.synchronize()
+    for i in range(n):
+        lo, hi = cu_seqlens_of(lens)[i], cu_seqlens_of(lens)[i + 1]
+        if lo == hi:
+            assert torch.equal(pool[i], pool0[i])
+            continue
+        one = [x[None, lo:hi].double().cpu() for x in ins]
+        y64, s64 = ow.wkv7_rowwise(*one, state=pool0[i][None].double().cpu())
+        assert close(y[lo:hi], y64[0], 2e-6) and close(pool[i], s64[0], 2e-6)
