@@ -317,6 +317,36 @@ int rwkv7_gemm_decode_partials(int64_t M, const void *A, const void *B, int64_t 
                                void *stream);
 
 /*
+ * A decode step of a bf16 model: every layer (rwkv7_shift_mix, rwkv7_gemm_decode /
+ * _partials, rwkv7_tmix_decode) and the final norm over M rows, in one call.
+ * `layers`: n_layer rows of pointers to the float32 vectors and packed weights
+ * those calls take; LoRA order w, a, g, v, layer 0 without v (NULL) and, past an
+ * embedding that is already normalised, without ln0.  kv [n_layer, S, C / 64, 64, 64],
+ * att_x and ffn_x [n_layer, S, C] are the slot pool.  out: [n_out, C] bf16, the
+ * ln_out rows logit_rows (NULL: rows 0 ..).  scratch: 256-byte aligned, of
+ * rwkv7_decode_layers_scratch bytes; ws: rwkv7_decode_layers_ws_floats floats.
+ */
+typedef struct rwkv7_layer {
+    const float *ln0_w, *ln0_b, *ln1_w, *ln1_b, *ln2_w, *ln2_b, *mix7, *mixk;
+    const float *tparams[8];
+    const void *r, *k, *v, *o, *fk, *fv;
+    const void *down[4], *up[4];
+    int64_t rank[4];
+} rwkv7_layer;
+int64_t rwkv7_decode_layers_scratch(int64_t M, int64_t C, int64_t FF, int n_layer,
+                                    const rwkv7_layer *layers);
+int64_t rwkv7_decode_layers_ws_floats(int64_t M, int64_t C, int64_t FF, int n_layer,
+                                      const rwkv7_layer *layers);
+int rwkv7_decode_layers(int64_t M, int64_t C, int64_t FF, int n_layer,
+                        const rwkv7_layer *layers, const int64_t *tokens,
+                        const void *emb, int64_t vocab, const int32_t *row_slot,
+                        const int32_t *row_last, float *kv, float *att_x, float *ffn_x,
+                        int64_t pool_slots, const float *ln_w, const float *ln_b,
+                        const int32_t *logit_rows, int64_t n_out, void *out,
+                        void *scratch, int64_t scratch_bytes, float *ws,
+                        int64_t ws_floats, void *stream);
+
+/*
  * Weight packing for rwkv7_gemm_decode: B [N][K] bf16 (row stride ldb, a
  * multiple of 8, K % 8 == 0) into rwkv7_gemm_packed_elems(N, K) bf16 elements
  * at `out`: 64 x 64 tiles of 8 KB, tile (nt, kt) at element

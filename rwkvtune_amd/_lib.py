@@ -62,6 +62,10 @@ SIGNATURES = {
     "rwkv7_gemm_decode_noalloc": (_I32, [_I64, _I32] + [_P] * 8 + [_P]),
     "rwkv7_gemm_decode_partial_count": (_I32, [_I64, _I32, _I32]),
     "rwkv7_gemm_decode_partials": (_I32, [_I64, _P, _P, _I64, _I32, _I32, _P, _I64, _P, _P]),
+    "rwkv7_decode_layers_scratch": (_I64, [_I64, _I64, _I64, _I32, _P]),
+    "rwkv7_decode_layers_ws_floats": (_I64, [_I64, _I64, _I64, _I32, _P]),
+    "rwkv7_decode_layers": (_I32, [_I64, _I64, _I64, _I32, _P, _P, _P, _I64] + [_P] * 5 + [_I64] + [_P] * 3
+                            + [_I64, _P, _P, _I64, _P, _I64, _P]),
     "rwkv7_gemm_packed_elems": (_I64, [_I32, _I32]),
     "rwkv7_gemm_pack": (_I32, [_P, _I64, _I32, _I32, _P, _P]),
     "rwkv7_head_logits": (_I32, [_I64, _I32, _I32, _P, _I64, _P, _P, _I64, _P]),
@@ -69,6 +73,14 @@ SIGNATURES = {
     "rwkv7_head_pack": (_I32, [_P, _I64, _I32, _I32, _P, _P]),
     "rwkv7_selective_log_softmax": (_I32, [_I32, _I64, _I64, _P, _I64, _P, _P, _P]),
 }
+
+
+class Layer(ctypes.Structure):
+    """``rwkv7_layer`` of ``rwkv7_hip.h``."""
+    _fields_ = ([(n, _P) for n in ("ln0_w", "ln0_b", "ln1_w", "ln1_b", "ln2_w", "ln2_b", "mix7", "mixk")]
+                + [("tparams", _P * 8)] + [(n, _P) for n in ("r", "k", "v", "o", "fk", "fv")]
+                + [("down", _P * 4), ("up", _P * 4), ("rank", _I64 * 4)])
+
 
 _lock = threading.Lock()
 _lib = None

@@ -111,6 +111,8 @@ bool misaligned(int dtype, const void* state, const void* r, const void* w, cons
 
 }  // namespace
 
+int capi_invalid(const char* msg) { return fail(RWKV7_ERR_INVALID, "%s", msg); }
+
 extern "C" int rwkv7_abi_version(void) { return 2; }
 
 extern "C" const char* rwkv7_last_error(void) { return g_err; }

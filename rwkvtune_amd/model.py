@@ -428,6 +428,26 @@ class _LayerPack:
                         self.gp[n] = PackedWeight(wt.detach())
                     else:
                         self.gp[n].pack(wt.detach())
+        if alloc and self.gp:
+            self.row = self._row()
+
+    def _row(self) -> _lib.Layer:
+        """The layer's row in the table of ``rwkv7_decode_layers`` (the buffers above
+        keep their addresses through ``refresh``)."""
+        p = lambda t: t.data_ptr()
+        row = _lib.Layer()
+        if self.ln0:
+            row.ln0_w, row.ln0_b = map(p, self.ln0)
+        row.ln1_w, row.ln1_b = map(p, self.ln1)
+        row.ln2_w, row.ln2_b = map(p, self.ln2)
+        row.mix7, row.mixk = p(self.mix7), p(self.mixk)
+        row.tparams = self.tparams
+        for n in ("r", "k", "v", "o", "fk", "fv"):
+            setattr(row, n, p(self.gp[n].t))
+        for i, n in enumerate(("w", "a", "g") if self.layer0 else ("w", "a", "g", "v")):
+            dn, up = self.gp[n + "1"], self.gp[n + "2"]
+            row.down[i], row.up[i], row.rank[i] = p(dn.t), p(up.t), dn.N
+        return row
 
 
 class RWKV7Model(nn.Module):
@@ -441,6 +461,7 @@ class RWKV7Model(nn.Module):
         self.ln_out = nn.LayerNorm(config.n_embd)
         self.head = nn.Linear(config.n_embd, config.vocab_size, bias=False)
         self._packs = None
+        self._rows = None
         self._head_pack = None
         self._packs_key = None
         self._packs_struct = None
@@ -512,7 +533,16 @@ class RWKV7Model(nn.Module):
         """(data_ptr, version) of every parameter: an in-place update (an
         optimizer step, ``copy_``, ``mul_`` ...) bumps the version, a move or
         reassignment changes the pointer."""
-        return tuple((p.data_ptr(), p._version) for p in self.parameters())
+        # (the modules' own dictionaries: parameters() builds every name on the way, 330 us of a
+        # 12-layer model's 430 us here)
+        key, stack = [], [self]
+        while stack:
+            m = stack.pop()
+            for p in m._parameters.values():
+                if p is not None:
+                    key.append((p.data_ptr(), p._version))
+            stack.extend(c for c in m._modules.values() if c is not None)
+        return tuple(key)
 
     def _struct_key(self):
         return (tuple((p.device, p.dtype, tuple(p.shape)) for p in self.parameters()),
@@ -540,6 +570,10 @@ class RWKV7Model(nn.Module):
                     self._head_pack.pack(self.head.weight.detach())
             else:
                 self._packs = [_LayerPack(b, C) for b in self.blocks]
+                # the layers' table of the native decode step (bf16 models)
+                self._rows = None
+                if self.dtype == torch.bfloat16:
+                    self._rows = (_lib.Layer * len(self._packs))(*[pk.row for pk in self._packs])
                 self._ln_out = (self.ln_out.weight.detach().float().contiguous(),
                                 self.ln_out.bias.detach().float().contiguous())
                 self._head_pack = None
@@ -666,6 +700,14 @@ class RWKV7Model(nn.Module):
         packs = self.packs()
         if M == 0:
             raise ValueError("forward_pooled needs at least one row")
+        n_out = M if logit_rows is None else (n_logit_rows if n_logit_rows is not None else logit_rows.numel())
+        # decode rows of a bf16 model use the grouped MFMA GEMM (small M, many
+        # projections); prefill and other dtypes use library GEMMs
+        grouped = decode and dt == torch.bfloat16 and self.use_grouped_gemm and M <= 1024
+        if (grouped and self.use_grouped_output and self._rows is not None and L > 0 and n_out > 0
+                and pool.kv.is_contiguous() and pool.att_x.is_contiguous() and pool.ffn_x.is_contiguous()):
+            xo = self._decode_layers(tokens, row_slot, row_last, pool, logit_rows, n_out, st)
+            return xo if return_hidden else self._head_logits(xo)
 
         x_res = torch.empty((M, C), dtype=torch.float32, device=dev)
         x_mid = torch.empty((M, C), dtype=torch.float32, device=dev)
@@ -683,9 +725,6 @@ class RWKV7Model(nn.Module):
         ffn_out = None
         ffn_parts, ffn_stride = 0, 0  # > 0: ffn_out holds the FFN value's float32 partial planes
         S = pool.n_slots
-        # decode rows of a bf16 model use the grouped MFMA GEMM (small M, many
-        # projections); prefill and other dtypes use library GEMMs
-        grouped = decode and dt == torch.bfloat16 and self.use_grouped_gemm and M <= 1024
         for l in range(L):
             blk = self.blocks[l]
             att, ffn, pk = blk.att, blk.ffn, packs[l]
@@ -774,7 +813,6 @@ class RWKV7Model(nn.Module):
                 _lib.call("rwkv7_activation", code, 2, hk.numel(), P(hk), st)
                 ffn_out = self._lin(hk, ffn.value.weight)
                 ffn_parts, ffn_stride = 0, 0
-        n_out = M if logit_rows is None else (n_logit_rows if n_logit_rows is not None else logit_rows.numel())
         if n_out == 0:
             return None
         xo = torch.empty((n_out, C), dtype=dt, device=dev)
@@ -783,6 +821,29 @@ class RWKV7Model(nn.Module):
         if return_hidden:
             return xo
         return self._head_logits(xo)
+
+    def _decode_layers(self, tokens, row_slot, row_last, pool, logit_rows, n_out, stream) -> torch.Tensor:
+        """Every layer and the final norm of a bf16 decode step, launched by one native
+        call (the same kernels and order as the loop of ``forward_pooled``): the
+        ``ln_out`` rows ``[n_out, n_embd]``."""
+        C, L, dev = self.config.n_embd, self.config.n_layer, tokens.device
+        M, FF = tokens.shape[0], self._packs[0].gp["fk"].N
+        lib, P, rows = _lib.load(), _lib.ptr, self._rows
+        nbytes = lib.rwkv7_decode_layers_scratch(M, C, FF, L, rows)
+        floats = lib.rwkv7_decode_layers_ws_floats(M, C, FF, L, rows)
+        if nbytes < 0 or floats < 0:
+            raise ValueError("rwkv7_decode_layers: " + lib.rwkv7_last_error().decode())
+        ws = self.gemm_workspace(dev)
+        ws.ensure(floats)
+        # 256-byte alignment whatever the allocator gives
+        scratch = torch.empty(nbytes + 255, dtype=torch.uint8, device=dev)
+        base = (scratch.data_ptr() + 255) // 256 * 256
+        xo = torch.empty((n_out, C), dtype=torch.bfloat16, device=dev)
+        _lib.call("rwkv7_decode_layers", M, C, FF, L, rows, P(tokens), P(self.emb.weight), self.config.vocab_size,
+                  P(row_slot), P(row_last), P(pool.kv), P(pool.att_x), P(pool.ffn_x), pool.n_slots,
+                  P(self._ln_out[0]), P(self._ln_out[1]), P(logit_rows), n_out, P(xo), base, nbytes, P(ws.ws),
+                  ws.ws.numel(), stream)
+        return xo
 
     def _head_logits(self, xo: torch.Tensor) -> torch.Tensor:
         """logits = head(xo) (model.py:494-495): the library's head GEMM over the
@@ -797,12 +858,32 @@ class RWKV7Model(nn.Module):
 
     @staticmethod
     def _meta_uniform(B: int, T: int, dev):
-        idx = torch.arange(B * T, dtype=torch.int32)
-        last = torch.full((B * T,), -1, dtype=torch.int32)
-        last[0::T] = idx[T - 1::T]
-        slot = (idx // T).to(torch.int32)
-        cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32)
-        return (slot.to(dev), last.to(dev), cu.to(dev), torch.arange(B, dtype=torch.int32).to(dev))
+        # built on the device: four host tensors cost four copies that each wait for the stream
+        seq = torch.arange(B, dtype=torch.int32, device=dev)
+        cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=dev)
+        if T == 1:
+            return seq, seq, cu, seq
+        slot = seq[:, None].expand(B, T).reshape(-1).contiguous()
+        last = torch.full((B * T,), -1, dtype=torch.int32, device=dev)
+        last[0::T] = cu[1:] - 1
+        return slot, last, cu, seq
+
+    def _pool_of(self, states, B: int) -> StatePool:
+        """A pool of ``B`` slots holding copies of per-layer states (``init_state``'s
+        layout; None: zeros)."""
+        cfg, dev = self.config, self.device
+        if states is None:
+            return StatePool(cfg, B, dev)
+        if len(states) != cfg.n_layer:
+            raise ValueError(f"expected {cfg.n_layer} layer states, got {len(states)}")
+        C, H = cfg.n_embd, cfg.n_head
+        f32 = dict(device=dev, dtype=torch.float32)
+        pool = StatePool.__new__(StatePool)
+        pool.n_slots = B
+        pool.att_x = torch.stack([s["att_x_prev"].reshape(B, C).to(**f32) for s in states])
+        pool.kv = torch.stack([s["att_kv"].reshape(B, H, HEAD_SIZE, HEAD_SIZE).to(**f32) for s in states])
+        pool.ffn_x = torch.stack([s["ffn_x_prev"].reshape(B, C).to(**f32) for s in states])
+        return pool
 
     @torch.no_grad()
     def forward_with_state(self, idx: torch.Tensor, states=None):
@@ -817,21 +898,13 @@ class RWKV7Model(nn.Module):
         if T == 0 or B == 0:
             raise ValueError("forward_with_state needs B > 0 and T > 0")
         dev = self.device
-        cfg = self.config
-        pool = StatePool(cfg, B, dev)
-        if states is not None:
-            if len(states) != cfg.n_layer:
-                raise ValueError(f"expected {cfg.n_layer} layer states, got {len(states)}")
-            for l, s in enumerate(states):
-                pool.att_x[l].copy_(s["att_x_prev"].reshape(B, -1))
-                pool.kv[l].copy_(s["att_kv"].reshape(pool.kv[l].shape))
-                pool.ffn_x[l].copy_(s["ffn_x_prev"].reshape(B, -1))
+        pool = self._pool_of(states, B)
         tokens = idx.to(device=dev, dtype=torch.int64).reshape(-1).contiguous()
         slot, last, cu, seq_slot = self._meta_uniform(B, T, dev)
         logits = self.forward_pooled(tokens, slot, last, pool, decode=(T == 1), cu_seqlens=cu,
                                      seq_slot=seq_slot)
-        new_states = [{"att_x_prev": pool.att_x[l], "att_kv": pool.kv[l], "ffn_x_prev": pool.ffn_x[l]}
-                      for l in range(cfg.n_layer)]
+        new_states = [{"att_x_prev": ax, "att_kv": kv, "ffn_x_prev": fx}
+                      for ax, kv, fx in zip(pool.att_x.unbind(0), pool.kv.unbind(0), pool.ffn_x.unbind(0))]
         return logits.view(B, T, -1), new_states
 
     @torch.no_grad()
@@ -928,14 +1001,7 @@ class RWKV7Model(nn.Module):
         ids = input_ids.to(device=dev, dtype=torch.int64)
         if n_new <= 0:
             return {"sequences": ids.clone()} if return_dict_in_generate else ids.clone()
-        pool = StatePool(cfg, B, dev)
-        if initial_states is not None:
-            if len(initial_states) != cfg.n_layer:
-                raise ValueError(f"expected {cfg.n_layer} layer states, got {len(initial_states)}")
-            for l, st in enumerate(initial_states):
-                pool.att_x[l].copy_(st["att_x_prev"].reshape(B, -1))
-                pool.kv[l].copy_(st["att_kv"].reshape(pool.kv[l].shape))
-                pool.ffn_x[l].copy_(st["ffn_x_prev"].reshape(B, -1))
+        pool = self._pool_of(initial_states, B)
         slot, last, cu, seq_slot = self._meta_uniform(B, T, dev)
         last_rows = (torch.arange(B, device=dev, dtype=torch.int32) * T + (T - 1)).contiguous()
         logits = self.forward_pooled(ids.reshape(-1).contiguous(), slot, last, pool, decode=(T == 1),
