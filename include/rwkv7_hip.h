@@ -410,6 +410,13 @@ int rwkv7_sample(int dtype, int64_t M, int64_t V, const void *logits, int64_t ld
                  const float *bias_val, const uint8_t *active, uint64_t seed,
                  const int64_t *rng_key, const int32_t *rng_ctr, int64_t *out_tok,
                  float *out_logp, void *stream);
+/* The same with one temperature, top_p, top_k and RNG key for every row (counter: the
+ * row's index), without per-row arrays. */
+int rwkv7_sample_uniform(int dtype, int64_t M, int64_t V, const void *logits, int64_t ld,
+                         int rule, int64_t max_valid_id, float temperature, float top_p,
+                         int top_k, const int32_t *bias_off, const int32_t *bias_ids,
+                         const float *bias_val, uint64_t seed, int64_t rng_key,
+                         int64_t *out_tok, float *out_logp, void *stream);
 
 /*
  * In-place repetition penalty on float32 logits [M, V] (row stride ld): for

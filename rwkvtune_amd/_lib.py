@@ -51,6 +51,8 @@ SIGNATURES = {
     "rwkv7_tmix_decode": (_I32, [_I32, _I64, _I64, _I32] + [_P] * 7 + [_P, _P, _P, _I64, _P, _P, _P]),
     "rwkv7_sample": (_I32, [_I32, _I64, _I64, _P, _I64, _I32, _I64, _P, _P, _P, _P, _P, _P, _P,
                             ctypes.c_uint64, _P, _P, _P, _P, _P]),
+    "rwkv7_sample_uniform": (_I32, [_I32, _I64, _I64, _P, _I64, _I32, _I64, ctypes.c_float, ctypes.c_float, _I32,
+                                    _P, _P, _P, ctypes.c_uint64, _I64, _P, _P, _P]),
     "rwkv7_repetition_penalty": (_I32, [_I64, _I64, _P, _I64, ctypes.c_float] + [_P] * 7 + [_P]),
     "rwkv7_rollout_first": (_I32, [_I64, _I64] + [_P] * 8 + [_I64, _I32, _P, _P]),
     "rwkv7_rollout_activate": (_I32, [_I64, _P, _I64, _I64] + [_P] * 8 + [_I64, _I32, _P, _P]),

@@ -387,8 +387,8 @@ extern "C" int rwkv7_tmix_decode(int dtype, int64_t M, int64_t H, int layer0, co
 // ---------------------------------------------------------------------------
 
 template <typename LT>
-hipError_t launch_sample(int M, int V, const void* logits, int64_t ld, int rule, int max_valid_id,
-                         const float* temperature, const float* top_p, const int32_t* top_k,
+hipError_t launch_sample(int M, int V, const void* logits, int64_t ld, int rule, int max_valid_id, float t, float p,
+                         int k, int64_t key, const float* temperature, const float* top_p, const int32_t* top_k,
                          const int32_t* bias_off, const int32_t* bias_ids, const float* bias_val,
                          const uint8_t* active, uint64_t seed, const int64_t* rng_key,
                          const int32_t* rng_ctr, int64_t* out_tok, float* out_logp, hipStream_t st);
@@ -398,43 +398,68 @@ hipError_t launch_rep_penalty(int M, int V, float* logits, int64_t ld, float pen
                               hipStream_t st);
 int sampler_max_vocab();
 
+namespace {
+// per-row arrays, or temperature == nullptr and t, p, k, key for every row
+int sample_rows(const char* fn, int dtype, int64_t M, int64_t V, const void* logits, int64_t ld, int rule,
+                int64_t max_valid_id, float t, float p, int k, int64_t key, const float* temperature, const float* top_p,
+                            const int32_t* top_k, const int32_t* bias_off, const int32_t* bias_ids,
+                            const float* bias_val, const uint8_t* active, uint64_t seed,
+                            const int64_t* rng_key, const int32_t* rng_ctr, int64_t* out_tok,
+                            float* out_logp, void* stream) {
+    if (!dtype_ok(dtype)) return fail(RWKV7_ERR_INVALID, "%s: bad dtype code %d", fn, dtype);
+    if (M < 0 || M > kMaxInt || V <= 0 || V > sampler_max_vocab() || ld < V)
+        return fail(RWKV7_ERR_INVALID, "%s: bad sizes M=%lld V=%lld ld=%lld (V <= %d)", fn, (long long)M,
+                    (long long)V, (long long)ld, sampler_max_vocab());
+    if (rule < 0 || rule > 2)
+        return fail(RWKV7_ERR_INVALID, "%s: rule must be 0 (batch), 1 (single) or 2 (generate)", fn);
+    if (M == 0) return ok();
+    if (!logits || !out_tok || !out_logp) return fail(RWKV7_ERR_INVALID, "%s: null pointer", fn);
+    if (bias_off != nullptr && (bias_ids == nullptr || bias_val == nullptr))
+        return fail(RWKV7_ERR_INVALID, "%s: bias_off needs bias_ids and bias_val", fn);
+    const int mv = max_valid_id < 0 ? (int)(V - 1) : (int)(max_valid_id < V ? max_valid_id : V - 1);
+    hipError_t e;
+    switch (dtype) {
+        case RWKV7_DTYPE_F32:
+            e = launch_sample<float>((int)M, (int)V, logits, ld, rule, mv, t, p, k, key, temperature, top_p, top_k, bias_off,
+                                     bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
+                                     (hipStream_t)stream);
+            break;
+        case RWKV7_DTYPE_F16:
+            e = launch_sample<f16_t>((int)M, (int)V, logits, ld, rule, mv, t, p, k, key, temperature, top_p, top_k, bias_off,
+                                     bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
+                                     (hipStream_t)stream);
+            break;
+        default:
+            e = launch_sample<bf16_t>((int)M, (int)V, logits, ld, rule, mv, t, p, k, key, temperature, top_p, top_k, bias_off,
+                                      bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
+                                      (hipStream_t)stream);
+            break;
+    }
+    return launch_status(e, "sample_kernel");
+}
+}  // namespace
+
 extern "C" int rwkv7_sample(int dtype, int64_t M, int64_t V, const void* logits, int64_t ld, int rule,
                             int64_t max_valid_id, const float* temperature, const float* top_p,
                             const int32_t* top_k, const int32_t* bias_off, const int32_t* bias_ids,
                             const float* bias_val, const uint8_t* active, uint64_t seed,
                             const int64_t* rng_key, const int32_t* rng_ctr, int64_t* out_tok,
                             float* out_logp, void* stream) {
-    if (!dtype_ok(dtype)) return fail(RWKV7_ERR_INVALID, "rwkv7_sample: bad dtype code %d", dtype);
-    if (M < 0 || M > kMaxInt || V <= 0 || V > sampler_max_vocab() || ld < V)
-        return fail(RWKV7_ERR_INVALID, "rwkv7_sample: bad sizes M=%lld V=%lld ld=%lld (V <= %d)", (long long)M,
-                    (long long)V, (long long)ld, sampler_max_vocab());
-    if (rule < 0 || rule > 2)
-        return fail(RWKV7_ERR_INVALID, "rwkv7_sample: rule must be 0 (batch), 1 (single) or 2 (generate)");
-    if (M == 0) return ok();
-    if (!logits || !temperature || !top_p || !top_k || !rng_key || !rng_ctr || !out_tok || !out_logp)
+    if (M > 0 && (!temperature || !top_p || !top_k || !rng_key || !rng_ctr))
         return fail(RWKV7_ERR_INVALID, "rwkv7_sample: null pointer");
-    if (bias_off != nullptr && (bias_ids == nullptr || bias_val == nullptr))
-        return fail(RWKV7_ERR_INVALID, "rwkv7_sample: bias_off needs bias_ids and bias_val");
-    const int mv = max_valid_id < 0 ? (int)(V - 1) : (int)(max_valid_id < V ? max_valid_id : V - 1);
-    hipError_t e;
-    switch (dtype) {
-        case RWKV7_DTYPE_F32:
-            e = launch_sample<float>((int)M, (int)V, logits, ld, rule, mv, temperature, top_p, top_k, bias_off,
-                                     bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
-                                     (hipStream_t)stream);
-            break;
-        case RWKV7_DTYPE_F16:
-            e = launch_sample<f16_t>((int)M, (int)V, logits, ld, rule, mv, temperature, top_p, top_k, bias_off,
-                                     bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
-                                     (hipStream_t)stream);
-            break;
-        default:
-            e = launch_sample<bf16_t>((int)M, (int)V, logits, ld, rule, mv, temperature, top_p, top_k, bias_off,
-                                      bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
-                                      (hipStream_t)stream);
-            break;
-    }
-    return launch_status(e, "sample_kernel");
+    return sample_rows("rwkv7_sample", dtype, M, V, logits, ld, rule, max_valid_id, 1.f, 1.f, 0, 0, temperature,
+                       top_p, top_k, bias_off, bias_ids, bias_val, active, seed, rng_key, rng_ctr, out_tok, out_logp,
+                       stream);
+}
+
+extern "C" int rwkv7_sample_uniform(int dtype, int64_t M, int64_t V, const void* logits, int64_t ld, int rule,
+                                    int64_t max_valid_id, float temperature, float top_p, int top_k,
+                                    const int32_t* bias_off, const int32_t* bias_ids, const float* bias_val,
+                                    uint64_t seed, int64_t rng_key, int64_t* out_tok, float* out_logp,
+                                    void* stream) {
+    return sample_rows("rwkv7_sample_uniform", dtype, M, V, logits, ld, rule, max_valid_id, temperature, top_p, top_k,
+                       rng_key, nullptr, nullptr, nullptr, bias_off, bias_ids, bias_val, nullptr, seed, nullptr,
+                       nullptr, out_tok, out_logp, stream);
 }
 
 extern "C" int rwkv7_repetition_penalty(int64_t M, int64_t V, float* logits, int64_t ld, float penalty,

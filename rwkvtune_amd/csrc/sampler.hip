@@ -789,9 +789,16 @@ __device__ __forceinline__ void walk_segment(HistShared& sh, unsigned long long 
     __syncthreads();
 }
 
+// One set of parameters for every row, where the per-row arrays are null (rng_ctr null: the row's index)
+struct SampleAll {
+    float temperature, top_p;
+    int top_k;
+    int64_t rng_key;
+};
+
 template <typename LT>
 __global__ __launch_bounds__(kT) void sample16_kernel(
-    int M, int V, const LT* __restrict__ logits, int64_t ld, int rule, int max_valid_id,
+    int M, int V, SampleAll all, const LT* __restrict__ logits, int64_t ld, int rule, int max_valid_id,
     const float* __restrict__ temperature, const float* __restrict__ top_p,
     const int32_t* __restrict__ top_k, const uint8_t* __restrict__ active, uint64_t seed,
     const int64_t* __restrict__ rng_key, const int32_t* __restrict__ rng_ctr, int64_t* __restrict__ out_tok,
@@ -802,7 +809,7 @@ __global__ __launch_bounds__(kT) void sample16_kernel(
     const int row = blockIdx.x;
     if (active != nullptr && active[row] == 0) return;  // whole block
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const float temp = temperature[row];
+    const float temp = temperature != nullptr ? temperature[row] : all.temperature;
     if (!(temp >= 1e-6f)) {  // greedy row (the counters' words serve as its reduction space)
         greedy_row<LT>(row, V, logits + (size_t)row * ld, max_valid_id, out_tok, out_logp, &red, sh.wm);
         return;
@@ -887,7 +894,8 @@ __global__ __launch_bounds__(kT) void sample16_kernel(
     block_scan2(inc_c, inc_m, sh, tc, tmx);
     const uint32_t exc_c = inc_c - own_c;
     const unsigned long long exc_m = inc_m - own_m;
-    const float u01 = uniform01(seed, (uint64_t)rng_key[row], (uint64_t)(uint32_t)rng_ctr[row]);
+    const float u01 = uniform01(seed, (uint64_t)(rng_key != nullptr ? rng_key[row] : all.rng_key),
+                                (uint64_t)(uint32_t)(rng_ctr != nullptr ? rng_ctr[row] : row));
     // (with a finite maximum the sum of q lies in [1, 65536]: only NaNs and
     // infinite maxima make the probabilities non-finite)
     const bool uniform = any_nan || !(mx > -INFINITY) || !(mx < INFINITY);
@@ -905,8 +913,8 @@ __global__ __launch_bounds__(kT) void sample16_kernel(
     }
 
     // kept: keys >= K, a prefix of the descending keys, with fixed-point mass Wfx
-    const int k = top_k[row];
-    const float p = top_p[row];
+    const int k = top_k != nullptr ? top_k[row] : all.top_k;
+    const float p = top_p != nullptr ? top_p[row] : all.top_p;
     const bool topk = k > 0 && k < V;
     const bool nucleus = p < 1.0f && (rule == RULE_BATCH || (rule == RULE_MIXIN && p > 0.f) ||
                                       (rule == RULE_SINGLE && k <= 0));
@@ -986,7 +994,7 @@ __global__ __launch_bounds__(kT) void sample16_kernel(
 
 template <typename LT>
 __global__ __launch_bounds__(kT) void sample_kernel(
-    int M, int V, const LT* __restrict__ logits, int64_t ld, int rule, int max_valid_id,
+    int M, int V, SampleAll all, const LT* __restrict__ logits, int64_t ld, int rule, int max_valid_id,
     const float* __restrict__ temperature, const float* __restrict__ top_p,
     const int32_t* __restrict__ top_k, const int32_t* __restrict__ bias_off,
     const int32_t* __restrict__ bias_ids, const float* __restrict__ bias_val,
@@ -1003,7 +1011,7 @@ __global__ __launch_bounds__(kT) void sample_kernel(
     const LT* lg = logits + (size_t)row * ld;
     const int vmax = max_valid_id < V - 1 ? max_valid_id : V - 1;
 
-    const float temp = temperature[row];
+    const float temp = temperature != nullptr ? temperature[row] : all.temperature;
     if (!(temp >= 1e-6f)) return;  // greedy rows belong to greedy_kernel
     float x[kVPT];
     load_row(lg, V, vmax, x);  // banned and padding: -inf
@@ -1028,8 +1036,8 @@ __global__ __launch_bounds__(kT) void sample_kernel(
         }
     }
 
-    const int k = top_k[row];
-    const float p = top_p[row];
+    const int k = top_k != nullptr ? top_k[row] : all.top_k;
+    const float p = top_p != nullptr ? top_p[row] : all.top_p;
     const bool topk = k > 0 && k < V;
     const bool nucleus = p < 1.0f && (rule == RULE_BATCH || (rule == RULE_MIXIN && p > 0.f) ||
                                       (rule == RULE_SINGLE && k <= 0));
@@ -1081,7 +1089,8 @@ __global__ __launch_bounds__(kT) void sample_kernel(
         lo = nlo > lo ? nlo : lo;
     }
 
-    draw_kept(key, lo, V, rule, uniform, uniform01(seed, (uint64_t)rng_key[row], (uint64_t)(uint32_t)rng_ctr[row]),
+    draw_kept(key, lo, V, rule, uniform, uniform01(seed, (uint64_t)(rng_key != nullptr ? rng_key[row] : all.rng_key),
+                                (uint64_t)(uint32_t)(rng_ctr != nullptr ? rng_ctr[row] : row)),
               fsum, &pick, sh, out_tok + row, out_logp + row);
 }
 
@@ -1095,7 +1104,7 @@ __global__ __launch_bounds__(kTG) void greedy_kernel(
     __shared__ unsigned long long red64[kWMax];
     const int row = blockIdx.x;
     if (active != nullptr && active[row] == 0) return;
-    if (temperature[row] >= 1e-6f) return;  // sampled rows belong to sample_kernel
+    if (temperature != nullptr && temperature[row] >= 1e-6f) return;  // sampled rows belong to sample_kernel
     greedy_row<LT>(row, V, logits + (size_t)row * ld, max_valid_id, out_tok, out_logp, &red, red64);
 }
 
@@ -1138,40 +1147,44 @@ __global__ __launch_bounds__(256) void rep_penalty_kernel(
 
 }  // namespace
 
+// temperature == nullptr: `t`, `p`, `k`, `key` for every row (one launch: the greedy or the sampling kernel)
 template <typename LT>
-hipError_t launch_sample(int M, int V, const void* logits, int64_t ld, int rule, int max_valid_id,
-                         const float* temperature, const float* top_p, const int32_t* top_k,
+hipError_t launch_sample(int M, int V, const void* logits, int64_t ld, int rule, int max_valid_id, float t, float p,
+                         int k, int64_t key, const float* temperature, const float* top_p, const int32_t* top_k,
                          const int32_t* bias_off, const int32_t* bias_ids, const float* bias_val,
                          const uint8_t* active, uint64_t seed, const int64_t* rng_key,
                          const int32_t* rng_ctr, int64_t* out_tok, float* out_logp, hipStream_t st)
 {
+    const SampleAll all = {t, p, k, key};
     if constexpr (sizeof(LT) == 2) {
         if (bias_off == nullptr) {  // one launch: sample16_kernel takes the greedy rows too
-            hipLaunchKernelGGL(sample16_kernel<LT>, dim3(M), dim3(kT), 0, st, M, V, (const LT*)logits, ld, rule,
+            hipLaunchKernelGGL(sample16_kernel<LT>, dim3(M), dim3(kT), 0, st, M, V, all, (const LT*)logits, ld, rule,
                                max_valid_id, temperature, top_p, top_k, active, seed, rng_key, rng_ctr, out_tok,
                                out_logp);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL(greedy_kernel<LT>, dim3(M), dim3(kTG), 0, st, M, V, (const LT*)logits, ld, max_valid_id,
-                       temperature, active, out_tok, out_logp);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sample_kernel<LT>, dim3(M), dim3(kT), 0, st, M, V, (const LT*)logits, ld, rule,
+    if (temperature != nullptr || !(t >= 1e-6f)) {
+        hipLaunchKernelGGL(greedy_kernel<LT>, dim3(M), dim3(kTG), 0, st, M, V, (const LT*)logits, ld, max_valid_id,
+                           temperature, active, out_tok, out_logp);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || temperature == nullptr) return e;
+    }
+    hipLaunchKernelGGL(sample_kernel<LT>, dim3(M), dim3(kT), 0, st, M, V, all, (const LT*)logits, ld, rule,
                        max_valid_id, temperature, top_p, top_k, bias_off, bias_ids, bias_val, active, seed,
                        rng_key, rng_ctr, out_tok, out_logp);
     return hipGetLastError();
 }
 
-template hipError_t launch_sample<float>(int, int, const void*, int64_t, int, int, const float*, const float*,
+template hipError_t launch_sample<float>(int, int, const void*, int64_t, int, int, float, float, int, int64_t, const float*, const float*,
                                          const int32_t*, const int32_t*, const int32_t*, const float*,
                                          const uint8_t*, uint64_t, const int64_t*, const int32_t*, int64_t*,
                                          float*, hipStream_t);
-template hipError_t launch_sample<bf16_t>(int, int, const void*, int64_t, int, int, const float*, const float*,
+template hipError_t launch_sample<bf16_t>(int, int, const void*, int64_t, int, int, float, float, int, int64_t, const float*, const float*,
                                           const int32_t*, const int32_t*, const int32_t*, const float*,
                                           const uint8_t*, uint64_t, const int64_t*, const int32_t*, int64_t*,
                                           float*, hipStream_t);
-template hipError_t launch_sample<f16_t>(int, int, const void*, int64_t, int, int, const float*, const float*,
+template hipError_t launch_sample<f16_t>(int, int, const void*, int64_t, int, int, float, float, int, int64_t, const float*, const float*,
                                          const int32_t*, const int32_t*, const int32_t*, const float*,
                                          const uint8_t*, uint64_t, const int64_t*, const int32_t*, int64_t*,
                                          float*, hipStream_t);

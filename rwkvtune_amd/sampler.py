@@ -52,16 +52,19 @@ class SamplerBuffers:
 
     def set_bias(self, logit_bias: Optional[dict], n_rows: int):
         """The same ``{token_id: bias}`` for every row (GRPO passes one dict)."""
-        if not logit_bias:
-            self.bias_off = self.bias_ids = self.bias_val = None
-            return
-        dev = self.temperature.device
-        ids = [int(k) for k in logit_bias.keys()]
-        vals = [float(v) for v in logit_bias.values()]
-        n = len(ids)
-        self.bias_ids = torch.tensor(ids * n_rows, dtype=torch.int32, device=dev)
-        self.bias_val = torch.tensor(vals * n_rows, dtype=torch.float32, device=dev)
-        self.bias_off = torch.arange(0, (n_rows + 1) * n, n, dtype=torch.int32, device=dev)
+        self.bias_off, self.bias_ids, self.bias_val = _bias_rows(logit_bias, n_rows, self.temperature.device)
+
+
+def _bias_rows(logit_bias: Optional[dict], n_rows: int, dev):
+    """CSR offsets, ids and values of one bias dict repeated for ``n_rows`` rows."""
+    if not logit_bias:
+        return None, None, None
+    ids = [int(k) for k in logit_bias.keys()]
+    vals = [float(v) for v in logit_bias.values()]
+    n = len(ids)
+    return (torch.arange(0, (n_rows + 1) * n, n, dtype=torch.int32, device=dev),
+            torch.tensor(ids * n_rows, dtype=torch.int32, device=dev),
+            torch.tensor(vals * n_rows, dtype=torch.float32, device=dev))
 
 
 def sample_rows(logits: torch.Tensor, buf: SamplerBuffers, *, rule: int, max_valid_id: Optional[int],
@@ -153,15 +156,17 @@ class TokenSampler:
             raise RuntimeError("TokenSampler runs on the GPU; logits must be a device tensor")
         logits2d = logits2d.contiguous()
         B = logits2d.shape[0]
-        buf = SamplerBuffers(B, logits2d.device)
-        buf.set_uniform(temperature, top_p, top_k)
-        buf.set_bias(logit_bias, B)
-        buf.rng_key.fill_(TokenSampler._next_key())
-        buf.rng_ctr.copy_(torch.arange(B, dtype=torch.int32, device=logits2d.device))
-        tok = torch.empty(B, dtype=torch.int64, device=logits2d.device)
-        lp = torch.empty(B, dtype=torch.float32, device=logits2d.device)
-        sample_rows(logits2d, buf, rule=rule, max_valid_id=TokenSampler._max_valid_token_id,
-                    seed=TokenSampler._seed, out_tok=tok, out_logp=lp)
+        dev, P = logits2d.device, _lib.ptr
+        if not -2 ** 31 <= int(top_k) < 2 ** 31:
+            raise RuntimeError(f"top_k {top_k} does not fit 32 bits")
+        mv = TokenSampler._max_valid_token_id
+        off, ids, val = _bias_rows(logit_bias, B, dev)
+        tok = torch.empty(B, dtype=torch.int64, device=dev)
+        lp = torch.empty(B, dtype=torch.float32, device=dev)
+        _lib.call("rwkv7_sample_uniform", _lib.dtype_code(logits2d.dtype), B, logits2d.shape[1], P(logits2d),
+                  logits2d.stride(0), rule, -1 if mv is None else int(mv), float(temperature), float(top_p),
+                  int(top_k), P(off), P(ids), P(val), ctypes_u64(TokenSampler._seed), TokenSampler._next_key(),
+                  P(tok), P(lp), _lib.stream_of(logits2d))
         return tok, lp
 
     @staticmethod
