@@ -99,13 +99,18 @@ int rwkv7_wkv_prefill(int dtype, int64_t nseq, int64_t H, int64_t total_tokens,
 
 /*
  * The same three calls with a float32 workspace (16-byte aligned; NULL or smaller
- * than rwkv7_wkv_segment_ws_floats: as without).  With it, 16-bit inputs of few
- * (sequence, head) pairs are walked in segments side by side instead of one block
- * per pair: the state recurrence of every segment first, then a scan over the
- * segments, then the full pass.  ragged = 0: nseq sequences of T tokens.
+ * than rwkv7_wkv_segment_ws_floats: as without).  With it, few (sequence, head)
+ * pairs are walked in segments side by side instead of one block per pair: the
+ * state recurrence of every segment first, then a scan over the segments, then the
+ * full pass.  kind: which call (UNIFORM and TRAIN: nseq sequences of T tokens).
  */
+enum {
+    RWKV7_SEGMENT_UNIFORM = 0, /* rwkv7s_forward_ws */
+    RWKV7_SEGMENT_RAGGED = 1,  /* rwkv7_wkv_prefill_ws */
+    RWKV7_SEGMENT_TRAIN = 2    /* rwkv7_wkv_train_forward_ws */
+};
 int64_t rwkv7_wkv_segment_ws_floats(int dtype, int64_t nseq, int64_t H, int64_t T,
-                                    int64_t total_tokens, int ragged);
+                                    int64_t total_tokens, int kind);
 int rwkv7s_forward_ws(int dtype, int64_t B, int64_t T, int64_t C, int64_t H, float *state,
                       const void *r, const void *w, const void *k, const void *v,
                       const void *a, const void *b, void *y, float *ws,

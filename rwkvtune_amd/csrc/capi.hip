@@ -18,7 +18,7 @@ hipError_t launch_wkv7_chunk(int nseq, int H, int T_uniform, const int32_t* cu_s
                              int pool_slots, int total_tokens, float* state, const void* r, const void* w,
                              const void* k, const void* v, const void* a, const void* b, void* y, float* ws,
                              int64_t ws_floats, hipStream_t stream);
-int64_t wkv7_chunk_ws(int nseq, int H, int T_uniform, bool ragged, int total, bool two_per_cu);
+int64_t wkv7_chunk_ws(int nseq, int H, int T_uniform, bool ragged, int total, bool two_per_cu, bool train);
 
 namespace {
 
@@ -118,13 +118,14 @@ extern "C" int rwkv7_abi_version(void) { return 2; }
 extern "C" const char* rwkv7_last_error(void) { return g_err; }
 
 extern "C" int64_t rwkv7_wkv_segment_ws_floats(int dtype, int64_t nseq, int64_t H, int64_t T, int64_t total_tokens,
-                                               int ragged) {
+                                               int kind) {
+    const bool ragged = kind == RWKV7_SEGMENT_RAGGED;
     ok();
     if (!dtype_ok(dtype) || nseq <= 0 || H <= 0 || total_tokens <= 0 ||
-        (ragged == 0 && T <= 0) || nseq * H > kMaxInt || T > kMaxInt || total_tokens > kMaxInt)
+        (!ragged && T <= 0) || nseq * H > kMaxInt || T > kMaxInt || total_tokens > kMaxInt)
         return 0;  // sizes that the call itself refuses or that have nothing to split
-    return wkv7_chunk_ws((int)nseq, (int)H, ragged ? 0 : (int)T, ragged != 0, (int)total_tokens,
-                         dtype == RWKV7_DTYPE_BF16);
+    return wkv7_chunk_ws((int)nseq, (int)H, ragged ? 0 : (int)T, ragged, (int)total_tokens,
+                         dtype == RWKV7_DTYPE_BF16, kind == RWKV7_SEGMENT_TRAIN);
 }
 
 extern "C" int rwkv7s_forward(int dtype, int64_t B, int64_t T, int64_t C, int64_t H, float* state,

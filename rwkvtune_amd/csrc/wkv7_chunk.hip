@@ -267,8 +267,15 @@ __device__ __forceinline__ float quad_bcast(float x, int e) {
 
 // Block barrier for data exchanged through LDS.  __syncthreads() also waits for every global load and store
 // of the wave: the loads issued a chunk ahead, y and the training checkpoints.  Training forward at
-// B = 8, T = 4096, H = 32 (bf16, one block per CU): 0.88 -> 0.73 ms; prefill the same either way.
+// B = 8, T = 4096, H = 32 (bf16, one block per CU): 0.88 -> 0.73 ms.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <bool LDS_ONLY>
+__device__ __forceinline__ void block_sync()
+{
+    if constexpr (LDS_ONLY) lds_barrier();
+    else __syncthreads();
+}
 
 // hi / lo bf16 parts of one value (hardware round-to-nearest-even)
 __device__ __forceinline__ void split1(float x, uint16_t& hi, uint16_t& lo) {
@@ -285,12 +292,13 @@ __device__ __forceinline__ void split1(float x, uint16_t& hi, uint16_t& lo) {
 // and the state after every 16th token of a sequence and after its last one
 // (ckpt [B][H][ceil(T/16)][64][64]), the layout the training backward reads.
 //
-// segs.cps > 0: the sequences are walked in segments (wkv7_seg.hpp), block group g taking segment g.  CARRY is
-// the pass before the scan: only the state is walked, blockIdx.y = 0 from the identity without values (M),
+// SEG: the sequences are walked in segments (wkv7_seg.hpp), block group g taking segment g (a template
+// argument, and the initial state's choice compiled only where there is one: the unsplit kernel lost 0.4 us a launch
+// to them).  CARRY is the pass before the scan: only the state is walked, blockIdx.y = 0 from the identity without values (M),
 // 1 from zero, or from the sequence's initial state in its first segment (N); the first segment's M place
 // keeps a copy of that initial state, since the last segment's block of the full pass writes the final state
 // where the first one's may still have to be read.
-template <typename IO, bool TRAIN = false, bool CARRY = false>
+template <typename IO, bool TRAIN, bool SEG, bool CARRY>
 __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) void wkv7_chunk2_kernel(
     int H, int T_uniform, const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ slot_idx, int pool_slots,
     int total_tokens, WkvSegs segs, float* seg_m, float* seg_n, float* state, const IO* __restrict__ r, const IO* __restrict__ w,
@@ -301,6 +309,10 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
     // bf16 inputs are exact as bf16 MFMA operands: V (unscaled) has no lo plane, and
     // the products with V skip their hi.lo term
     constexpr bool kVExact = std::is_same<IO, bf16_t>::value;
+    // The next chunk's loads: with the training stores in flight, early and behind barriers that wait for LDS only;
+    // the prefill kernel (two blocks per CU) is 0.5-1 % faster with them late (27 ragged sequences, H = 16:
+    // 39.1 -> 38.6 us; 16 x 300, H = 32: 67.1 -> 66.9).
+    constexpr bool kFetchB = TRAIN;
     constexpr int kVLo = kVExact ? 0 : 1;  // plane of V's lo part (none for bf16)
     __shared__ ChunkLds2<!kVExact> sm;
     const int unit = blockIdx.x;
@@ -319,7 +331,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
     int s = unit / H;
     int seg = 0, nsg = 1;  // segment of the sequence
     const bool ident = CARRY && blockIdx.y == 0;
-    if (segs.cps > 0) {
+    if constexpr (SEG) {
         if (!wkvseg::locate(segs, unit / H, s, seg, nsg)) return;
         if (CARRY && (seg == nsg - 1 || (ident && seg == 0))) return;
     } else if (cu_seqlens != nullptr) {
@@ -327,7 +339,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         if (nseq <= 256) {
             int* lens = sm.u.lens;
             for (int c = tid; c < nseq; c += 256) lens[c] = cu_seqlens[c + 1] - cu_seqlens[c];
-            lds_barrier();
+            block_sync<kFetchB>();
             for (int c = tid; c < nseq; c += 256) {
                 const int len = lens[c];
                 int rank = 0;
@@ -337,7 +349,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 }
                 if (rank == s) sm.pick = c;
             }
-            lds_barrier();
+            block_sync<kFetchB>();
             s = sm.pick;
         }
     }
@@ -374,14 +386,18 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             }
         }
     };
-    // the initial state of the sequence: the pool slot's, or (training) s_init
-    const float* gInit = s_init != nullptr ? s_init + ((size_t)s * H + h) * (NH * NH) : TRAIN ? nullptr : gS;
-    if (seg > 0 || (nsg > 1 && !CARRY))  // found by the passes before (unused in CARRY)
-        gInit = seg > 0 ? seg_n + (size_t)(unit - H) * (NH * NH) : seg_m + (size_t)unit * (NH * NH);
-    if (gInit == nullptr || (CARRY && seg > 0))
-        tile = f32x16{0.f};
-    else
-        tile_io(const_cast<float*>(gInit), NH, false);
+    if constexpr (!SEG && !TRAIN) {
+        tile_io(gS, NH, false);
+    } else {
+        // the initial state of the sequence: the pool slot's, or (training) s_init
+        const float* gInit = s_init != nullptr ? s_init + ((size_t)s * H + h) * (NH * NH) : TRAIN ? nullptr : gS;
+        if (SEG && (seg > 0 || (nsg > 1 && !CARRY)))  // found by the passes before (unused in CARRY)
+            gInit = seg > 0 ? seg_n + (size_t)(unit - H) * (NH * NH) : seg_m + (size_t)unit * (NH * NH);
+        if (gInit == nullptr || (CARRY && seg > 0))
+            tile = f32x16{0.f};
+        else
+            tile_io(const_cast<float*>(gInit), NH, false);
+    }
     if (CARRY && seg == 0) tile_io(seg_m + (size_t)unit * (NH * NH), NH, true);
     if (ident) {
 #pragma unroll
@@ -424,7 +440,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         if (ident) raw[3][0] = raw[3][1] = make_uint2(0, 0);
     };
     // the tokens this block walks
-    const int t_lo = tb + seg * segs.cps * L, t_hi = nsg > 1 ? min(te, t_lo + segs.cps * L) : te;
+    const int t_lo = SEG ? tb + seg * segs.cps * L : tb, t_hi = SEG && nsg > 1 ? min(te, t_lo + segs.cps * L) : te;
     fetch(t_lo);
 
     for (int t0 = t_lo; t0 < t_hi; t0 += L) {
@@ -459,7 +475,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
         if (g == 3) *reinterpret_cast<f32x4*>(&sm.tot[wave][j0]) = inc;
         const bool wave_slow = __ballot(slow) != 0;
         if (lane == 0) sm.slow[wave] = wave_slow ? 1 : 0;
-        lds_barrier();
+        block_sync<kFetchB>();
         const int4 sl = *reinterpret_cast<const int4*>(sm.slow);
         const bool any_slow = (sl.x | sl.y | sl.z | sl.w) != 0;
 
@@ -542,12 +558,12 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 }
             }
         }
-        lds_barrier();
+        block_sync<kFetchB>();
 
         if (any_slow) {
             // ---- exact token-serial update on a float32 copy of the state in LDS ----
             tile_io(&sm.u.Sf[0][0], SP, true);
-            lds_barrier();
+            block_sync<kFetchB>();
             const int i = tid >> 2, q = tid & 3;
             for (int t = 0; t < n; ++t) {
                 const size_t off = (size_t)(t0 + t) * C + h * NH;
@@ -580,7 +596,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                     }
                 }
             }
-            lds_barrier();
+            block_sync<kFetchB>();
             // back to the registers, and the hi/lo planes
             tile_io(&sm.u.Sf[0][0], SP, false);
             store_state_planes(&sm.Sp[0][0][0], ir_t, jt_t, tile, lane);
@@ -589,9 +605,8 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
             continue;
         }
 
-        // the raw registers are free from here to the next phase A: fetch the next chunk (LDS barriers do not
-        // wait for global loads, so these stay in flight through phases B to D)
-        if (t0 + L < t_hi) fetch(t0 + L);
+        // the raw registers are free from here to the next phase A
+        if (kFetchB && t0 + L < t_hi) fetch(t0 + L);
 
         // ---- B: two 32x32 tiles per wave, K = 64 over keys, sharing one operand:
         //   wave 0: X (value tile 0) and A_ab,   wave 1: X (value tile 1) and A_ak,
@@ -637,7 +652,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 c1[q] = keep ? c1[q] : 0.f;
             }
             // the products overwrite the planes they were computed from
-            lds_barrier();
+            block_sync<kFetchB>();
             if (wave == kA) {
                 float* AT = &sm.u.pb.AT[0][0];
 #pragma unroll
@@ -650,7 +665,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 store_planes_T(out, TQ, T32_PLANE, 0, 0, c1, lane);
             }
         }
-        lds_barrier();
+        block_sync<kFetchB>();
 
         // ---- C: X += V^T A_ak (waves 0/1), stored as X^T; Y += V^T B_rk (waves 2/3) --
         if (!CARRY || wave < 2) {
@@ -671,7 +686,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                 *reinterpret_cast<f32x4*>(XT + xtswz(t, 32 * wave + 8 * g + 4 * (lane >> 5))) =
                     f32x4{accXY[4 * g], accXY[4 * g + 1], accXY[4 * g + 2], accXY[4 * g + 3]};
         }
-        lds_barrier();
+        block_sync<kFetchB>();
 
         // ---- triangular solve: SA[i][t] = X[i][t] + sum_{u<t} SA[i][u] A_ab[u][t] -----
         // Right-looking: lane q of row i keeps running sums for its targets t = 4m + q.
@@ -746,7 +761,9 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
                     if (4 * m + q < n) sa_out[(size_t)(t0 + 4 * m + q) * C + h * NH + i] = pq[m];
             }
         }
-        lds_barrier();
+        block_sync<kFetchB>();
+
+        if (!kFetchB && t0 + L < t_hi) fetch(t0 + L);
 
         // ---- D: every wave: its state tile += (b^^T SA)^T, scaled by D_L and stored as the next chunk's
         //         planes; waves 2/3 also Y += SA B_rb (value tile wave - 2) and store y
@@ -810,7 +827,7 @@ __global__ __launch_bounds__(256, (std::is_same<IO, bf16_t>::value ? 2 : 1)) voi
     if constexpr (CARRY) {
         tile_io((ident ? seg_m : seg_n) + (size_t)unit * (NH * NH), NH, true);
     } else {
-        if (gS != nullptr && seg == nsg - 1) tile_io(gS, NH, true);
+        if ((!TRAIN || gS != nullptr) && (!SEG || seg == nsg - 1)) tile_io(gS, NH, true);
     }
 }
 
@@ -831,23 +848,25 @@ hipError_t launch_wkv7_fwd32(const WkvSegs& m, int H, int T_uniform, const int32
                              float* sa, float* ws, hipStream_t stream);
 
 // Segments of a launch; cps = 0 (unsplit) where that is not slower.  n segments per sequence cost the state
-// pass (0.75 of a full walk per chunk; 2 n - 3 blocks per unit), the scan (0.5 us a step) and the full pass
-// over n segments, against one block per unit over the whole sequence.  Ragged sequences count with their
-// average length.  Measured (us, bf16, unsplit -> split): 12 units 128 tokens 22 -> 20, 12 x 512 76 -> 31,
-// 32 x 1000 148 -> 54, 32 x 4096 580 -> 150, 64 x 256 40 -> 35, 64 x 2048 291 -> 146, 128 x 1000 148 -> 131;
-// not split by the model and slower split: 32 x 64 13 -> 18, 64 x 160 27 -> 30, 128 x 384 58 -> 60,
-// 192 x 4096 583 -> 679, 256 x 4096 588 -> 744.
-static WkvSegs plan_segments(int nseq, int H, int T_uniform, const int32_t* cu, int total, bool two_per_cu)
+// pass (0.75 of a full walk per chunk; 2 n - 3 blocks per unit), the scan (0.5 us a step), two more launches and
+// the full pass over n segments, against one block per unit over the whole sequence.  Two launches are 9 us on the
+// device; in the training operator, where a call this small waits for its caller (110 us of autograd for 20 of
+// kernels), also what they cost the caller, 18 us.  Ragged sequences count with their average length, and unsplit
+// with a quarter more: the launch ends with its longest one.  Measured (us, bf16, unsplit -> split): 12 units
+// 128 tokens 22 -> 20, 12 x 512 76 -> 31, 32 x 1000 148 -> 54, 32 x 4096 580 -> 150, 64 x 256 40 -> 35,
+// 64 x 2048 291 -> 146, 128 x 1000 148 -> 131, 60 ragged of 83 - 322 49 -> 41; not split by the model and slower
+// split: 32 x 64 13 -> 18, 64 x 160 27 -> 30, 128 x 384 58 -> 60, 192 x 4096 583 -> 679, 256 x 4096 588 -> 744.
+static WkvSegs plan_segments(int nseq, int H, int T_uniform, const int32_t* cu, int total, bool two_per_cu, bool train)
 {
     WkvSegs m = {nseq, 0, 0, T_uniform, total, cu};
     const int64_t units = (int64_t)nseq * H;
     const int per_seq = cu == nullptr ? (T_uniform + L - 1) / L : (int)(((int64_t)total + nseq * L - 1) / ((int64_t)nseq * L));
     if (units >= 256) return m;
-    float best = per_seq * walk_cost(units, two_per_cu);
+    float best = (cu == nullptr || nseq == 1 ? 1.f : 1.25f) * per_seq * walk_cost(units, two_per_cu);
     for (int n = 2; n <= 32 && n <= per_seq; ++n) {
         const int cps = (per_seq + n - 1) / n, nn = (per_seq + cps - 1) / cps;
         const float cost = cps * (0.75f * walk_cost(units * (2 * nn - 3), two_per_cu) +
-                                  walk_cost(units * nn, two_per_cu)) + 0.5f * nn + 9.f;
+                                  walk_cost(units * nn, two_per_cu)) + 0.5f * nn + (train ? 18.f : 9.f);
         if (cost < best) {
             best = cost;
             m.cps = cps;
@@ -858,12 +877,11 @@ static WkvSegs plan_segments(int nseq, int H, int T_uniform, const int32_t* cu, 
     return m;
 }
 
-// floats of workspace with which a 16-bit launch of these sizes may run in segments (cu: any non-null
-// pointer for ragged sequences); without it, it runs unsplit
-int64_t wkv7_chunk_ws(int nseq, int H, int T_uniform, bool ragged, int total, bool two_per_cu)
+// floats of workspace with which a launch of these sizes may run in segments; without it, it runs unsplit
+int64_t wkv7_chunk_ws(int nseq, int H, int T_uniform, bool ragged, int total, bool two_per_cu, bool train)
 {
     static const int32_t some = 0;
-    const WkvSegs m = plan_segments(nseq, H, T_uniform, ragged ? &some : nullptr, total, two_per_cu);
+    const WkvSegs m = plan_segments(nseq, H, T_uniform, ragged ? &some : nullptr, total, two_per_cu, train);
     return (int64_t)m.gmax * H * 2 * NH * NH;
 }
 
@@ -873,24 +891,24 @@ static hipError_t launch_chunk2(int nseq, int H, int T_uniform, const int32_t* c
                                 const void* v, const void* a, const void* b, void* y, const float* s0, float* ckpt,
                                 float* sa, float* ws, int64_t ws_floats, hipStream_t stream)
 {
-    WkvSegs m = plan_segments(nseq, H, T_uniform, cu_seqlens, total, std::is_same<IO, bf16_t>::value);
+    WkvSegs m = plan_segments(nseq, H, T_uniform, cu_seqlens, total, std::is_same<IO, bf16_t>::value, TRAIN);
     const int64_t half = (int64_t)m.gmax * H * NH * NH;
     if (m.cps > 0 && (ws == nullptr || ws_floats < 2 * half)) m.cps = 0;
     float *sm = ws, *sn = ws + half;
     const unsigned groups = m.cps > 0 ? (unsigned)m.gmax : (unsigned)nseq;
-    if (m.cps > 0) {
-        hipLaunchKernelGGL((wkv7_chunk2_kernel<IO, false, true>), dim3(groups * (unsigned)H, 2), dim3(256), 0, stream,
-                           H, T_uniform, cu_seqlens, slot_idx, pool_slots, total, m, sm, sn, TRAIN ? nullptr : state,
-                           (const IO*)r, (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a, (const IO*)b,
-                           (IO*)y, s0, nullptr, nullptr);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = launch_wkv7_scan_forward(m, H, sm, sn, stream);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL((wkv7_chunk2_kernel<IO, TRAIN, false>), dim3(groups * (unsigned)H), dim3(256), 0, stream, H,
-                       T_uniform, cu_seqlens, slot_idx, pool_slots, total, m, sm, sn, state, (const IO*)r,
-                       (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a, (const IO*)b, (IO*)y, s0, ckpt, sa);
-    return hipGetLastError();
+    auto walk = [&](auto kern, dim3 grid, float* st, float* ck, float* sa_) -> hipError_t {
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, H, T_uniform, cu_seqlens, slot_idx, pool_slots, total, m,
+                           sm, sn, st, (const IO*)r, (const IO*)w, (const IO*)k, (const IO*)v, (const IO*)a,
+                           (const IO*)b, (IO*)y, s0, ck, sa_);
+        return hipGetLastError();
+    };
+    const dim3 grid(groups * (unsigned)H);
+    if (m.cps == 0) return walk(wkv7_chunk2_kernel<IO, TRAIN, false, false>, grid, state, ckpt, sa);
+    hipError_t e = walk(wkv7_chunk2_kernel<IO, false, true, true>, dim3(grid.x, 2), TRAIN ? nullptr : state, nullptr,
+                        nullptr);
+    if (e == hipSuccess) e = launch_wkv7_scan_forward(m, H, sm, sn, stream);
+    if (e != hipSuccess) return e;
+    return walk(wkv7_chunk2_kernel<IO, TRAIN, true, false>, grid, state, ckpt, sa);
 }
 
 template <typename IO>
@@ -900,7 +918,7 @@ hipError_t launch_wkv7_chunk(int nseq, int H, int T_uniform, const int32_t* cu_s
                              int64_t ws_floats, hipStream_t stream)
 {
     if constexpr (sizeof(IO) == 4) {
-        WkvSegs m = plan_segments(nseq, H, T_uniform, cu_seqlens, total_tokens, false);
+        WkvSegs m = plan_segments(nseq, H, T_uniform, cu_seqlens, total_tokens, false, false);
         if (ws == nullptr || ws_floats < (int64_t)m.gmax * H * 2 * NH * NH) m.cps = 0;
         return launch_wkv7_fwd32(m, H, T_uniform, cu_seqlens, slot_idx, pool_slots, total_tokens, state,
                                  (const float*)r, (const float*)w, (const float*)k, (const float*)v, (const float*)a,
@@ -920,7 +938,7 @@ hipError_t launch_wkv7_chunk_train(int B, int T, int H, const void* r, const voi
                                    float* sa, float* ws, int64_t ws_floats, hipStream_t stream)
 {
     if constexpr (sizeof(IO) == 4) {
-        WkvSegs m = plan_segments(B, H, T, nullptr, B * T, false);
+        WkvSegs m = plan_segments(B, H, T, nullptr, B * T, false, true);
         if (ws == nullptr || ws_floats < (int64_t)m.gmax * H * 2 * NH * NH) m.cps = 0;
         return launch_wkv7_fwd32(m, H, T, nullptr, nullptr, B, B * T, s_out, (const float*)r, (const float*)w,
                                  (const float*)k, (const float*)v, (const float*)a, (const float*)b, (float*)y, s0,

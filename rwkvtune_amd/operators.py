@@ -41,6 +41,7 @@ The reference's loader names (``load_cuda_operator_*``) are aliases here.
 
 from __future__ import annotations
 
+import functools
 import os
 import threading
 from typing import Callable
@@ -79,10 +80,21 @@ def _contig(*ts):
     return out
 
 
-def _segment_ws(dtype, nseq, H, T, total, ragged, device):
+@functools.lru_cache(maxsize=256)  # a function of the sizes alone
+def _segment_floats(dtype, nseq, H, T, total, kind):
+    return _lib.load().rwkv7_wkv_segment_ws_floats(_lib.dtype_code(dtype), nseq, H, T, total, kind)
+
+
+@functools.lru_cache(maxsize=256)
+def _backward_floats(B, T, H):
+    return _lib.load().rwkv7_wkv_train_backward_ws_floats(B, T, H)
+
+
+def _segment_ws(dtype, nseq, H, T, total, kind, device):
     """``(workspace tensor or None, floats)`` with which a chunked call of few
-    (sequence, head) pairs walks its sequences in segments side by side."""
-    n = _lib.load().rwkv7_wkv_segment_ws_floats(_lib.dtype_code(dtype), nseq, H, T, total, int(ragged))
+    (sequence, head) pairs walks its sequences in segments side by side; ``kind``:
+    0 uniform, 1 ragged, 2 the training forward."""
+    n = _segment_floats(dtype, nseq, H, T, total, kind)
     return (torch.empty(n, dtype=torch.float32, device=device), n) if n > 0 else (None, 0)
 
 
@@ -111,7 +123,7 @@ def wkv7s_forward(state, r, w, k, v, a, b, head_size: int = HEAD_SIZE):
         raise RuntimeError(f"state must be a contiguous [B={B}, H={H}, {head_size}, {head_size}] tensor")
     r, w, k, v, a, b = _contig(r, w, k, v, a, b)
     y = torch.empty(r.shape, dtype=r.dtype, device=r.device)
-    ws, n = _segment_ws(r.dtype, B, H, T, B * T, False, r.device)
+    ws, n = _segment_ws(r.dtype, B, H, T, B * T, 0, r.device)
     _lib.call("rwkv7s_forward_ws", _lib.dtype_code(r.dtype), B, T, C, H, _lib.ptr(state),
               *(_lib.ptr(t) for t in (r, w, k, v, a, b)), _lib.ptr(y), _lib.ptr(ws), n, _lib.stream_of(r))
     return y
@@ -162,7 +174,7 @@ def _train_forward(w, q, k, v, a, b, s0=None, s_out=None):
     ckpt = torch.empty((B, H, nck, N, N), dtype=torch.float32, device=dev)
     sa = torch.empty((B, T, H, N), dtype=torch.float32, device=dev)
     P = _lib.ptr
-    ws, n = _segment_ws(q.dtype, B, H, T, B * T, False, dev)
+    ws, n = _segment_ws(q.dtype, B, H, T, B * T, 2, dev)
     _lib.call("rwkv7_wkv_train_forward_ws", _lib.dtype_code(q.dtype), B, T, H, P(q), P(w), P(k), P(v), P(a), P(b),
               P(y), P(s0), P(s_out), P(ckpt), P(sa), P(ws), n, _lib.stream_of(q))
     return y, ckpt, sa
@@ -172,7 +184,7 @@ def _train_backward(w, q, k, v, a, b, dy, ckpt, sa, ds_in=None, want_ds0=False, 
     """``start_known``: ``s0`` (None: zero) is the forward's initial state; otherwise
     it is recovered from the first checkpoint."""
     B, T, H, N = q.shape
-    need = _lib.load().rwkv7_wkv_train_backward_ws_floats(B, T, H)
+    need = _backward_floats(B, T, H)
     ws = torch.empty(need, dtype=torch.float32, device=q.device) if need > 0 else None
     grads = [torch.empty_like(x) for x in (w, q, k, v, a, b)]
     dw, dq, dk, dv, da, db = grads
@@ -399,7 +411,7 @@ def wkv7_prefill(state_pool, slot_idx, cu_seqlens, r, w, k, v, a, b, y=None, chu
         y = torch.empty(r.shape, dtype=r.dtype, device=r.device)
     _check_out(y, r)
     ins = _contig(r, w, k, v, a, b)  # kept alive until the launch is enqueued
-    ws, n = _segment_ws(r.dtype, nseq, H, 0, total, True, r.device)
+    ws, n = _segment_ws(r.dtype, nseq, H, 0, total, 1, r.device)
     _lib.call("rwkv7_wkv_prefill_ws", _lib.dtype_code(r.dtype), nseq, H, total,
               _lib.ptr(cu_seqlens), _lib.ptr(slot_idx), _lib.ptr(state_pool), S,
               *(_lib.ptr(t) for t in ins), _lib.ptr(y), int(chunk_len), _lib.ptr(ws), n, _lib.stream_of(r))

@@ -39,7 +39,7 @@ def unsplit_prefill(pool, slot, cu, ins, total):
 def test_ragged_prefill(gpu_device, dtype, H, lens):
     print(f"[case] segmented prefill {dtype} H={H} lens={lens}", flush=True)
     total, n = sum(lens), len(lens)
-    assert ops._segment_ws(dtype, n, H, 0, total, True, gpu_device)[1] > 0
+    assert ops._segment_ws(dtype, n, H, 0, total, 1, gpu_device)[1] > 0
     ins = [x.to(gpu_device) for x in wkv_inputs((total,), H, seed=total, dtype=dtype).as_tuple()]
     ins[1][total // 2, 5] = 1.0  # a chunk below the matrix form's log-decay floor
     cu = torch.tensor(cu_seqlens_of(lens), dtype=torch.int32, device=gpu_device)
@@ -81,7 +81,7 @@ def test_training_forward(gpu_device, B, T, H, alias):
     """y, sa, checkpoints and the final state; the final state may be written over the initial one."""
     print(f"[case] segmented training forward B={B} T={T} H={H} alias={alias}", flush=True)
     dtype = torch.bfloat16
-    assert ops._segment_ws(dtype, B, H, T, B * T, False, gpu_device)[1] > 0
+    assert ops._segment_ws(dtype, B, H, T, B * T, 2, gpu_device)[1] > 0
     xs = [x.view(B, T, H, 64).to(gpu_device) for x in wkv_inputs((B, T), H, seed=T, dtype=dtype).as_tuple()]
     r, w, k, v, a, b = xs
     s0 = wkv_state(B, H).to(gpu_device)
@@ -101,7 +101,7 @@ def test_workspace_too_small_runs_unsplit(gpu_device):
     H, T = 4, 512
     print("[case] segmented prefill, small workspace", flush=True)
     ins = [x.to(gpu_device) for x in wkv_inputs((1, T), H, seed=9).as_tuple()]
-    need = ops._segment_ws(torch.bfloat16, 1, H, T, T, False, gpu_device)[1]
+    need = ops._segment_ws(torch.bfloat16, 1, H, T, T, 0, gpu_device)[1]
     ws = torch.empty(need - 1, dtype=torch.float32, device=gpu_device)
     s1, s2 = wkv_state(1, H).to(gpu_device), wkv_state(1, H).to(gpu_device)
     y1, y2 = torch.empty_like(ins[0]), torch.empty_like(ins[0])
