@@ -34,7 +34,7 @@ struct __attribute__((aligned(16))) FwdLds {
     float T[L][TP], AbT[L][TP], Rb[L][TP], Ak[L][TP], Rk[L][TP];  // AbT [t][s], the others [s][t]
     double tot[NW][NH];
     float D15[NH];
-    int slow[NW];
+    alignas(16) int slow[NW];
 };
 
 // TRAIN, CARRY, segs, seg_m, seg_n, s_init, ckpt, sa_out: as wkv7_chunk2_kernel (wkv7_chunk.hip)
@@ -46,8 +46,7 @@ __global__ __launch_bounds__(TH) void wkv7_fwd32_kernel(
     const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ y, const float* s_init,
     float* __restrict__ ckpt, float* __restrict__ sa_out)
 {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    FwdLds& sm = *reinterpret_cast<FwdLds*>(smem);
+    __shared__ FwdLds sm;
     const int tid = threadIdx.x, lane0 = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int unit = blockIdx.x, h = unit % H;
@@ -130,7 +129,10 @@ __global__ __launch_bounds__(TH) void wkv7_fwd32_kernel(
         lds_barrier();
         int any_slow = 0;
 #pragma unroll
-        for (int q = 0; q < NW; ++q) any_slow |= sm.slow[q];
+        for (int q = 0; q < NW; q += 4) {
+            const int4 x = *reinterpret_cast<const int4*>(&sm.slow[q]);
+            any_slow |= x.x | x.y | x.z | x.w;
+        }
 
         if (any_slow) {
             // ---- exact token-serial update: 16 threads per state row, four columns each --------------
@@ -176,12 +178,17 @@ __global__ __launch_bounds__(TH) void wkv7_fwd32_kernel(
         }
 
         // ---- scaled operands -----------------------------------------------------------------------
+        // (all reads first: a branch around each would wait for them one by one)
+        double tots[NW - 1][2];
 #pragma unroll
         for (int q = 0; q < NW - 1; ++q) {
-            if (q < wave) {  // uniform
-                before[0] += sm.tot[q][j0];
-                before[1] += sm.tot[q][j0 + 1];
-            }
+            tots[q][0] = sm.tot[q][j0];
+            tots[q][1] = sm.tot[q][j0 + 1];
+        }
+#pragma unroll
+        for (int q = 0; q < NW - 1; ++q) {
+            before[0] += q < wave ? tots[q][0] : 0.0;
+            before[1] += q < wave ? tots[q][1] : 0.0;
         }
         float D15[2];
 #pragma unroll
@@ -330,10 +337,7 @@ hipError_t launch_wkv7_fwd32(const WkvSegs& m, int H, int T_uniform, const int32
     const unsigned groups = m.cps > 0 ? (unsigned)m.gmax : (unsigned)m.nseq;
     float *sm = ws, *sn = m.cps > 0 ? ws + (size_t)m.gmax * H * NH * NH : nullptr;
     auto launch = [&](auto kern, dim3 grid, float* st, float* ck, float* sa_) -> hipError_t {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(FwdLds));
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, grid, dim3(TH), sizeof(FwdLds), stream, H, T_uniform, cu, slot_idx, pool_slots, total,
+        hipLaunchKernelGGL(kern, grid, dim3(TH), 0, stream, H, T_uniform, cu, slot_idx, pool_slots, total,
                            m, sm, sn, st, r, w, k, v, a, b, y, s0, ck, sa_);
         return hipGetLastError();
     };

@@ -69,7 +69,7 @@ struct __attribute__((aligned(16))) BwdLds {
     float G[NH][SP];                        // G^ of the chunk [i][j]
     float T[L][TP], AbT[L][TP], Rb[L][TP];  // T [s][t], A_ab^T [t][s], B_rb [s][t]
     DT tot[GRADS ? 16 : 8][NH];
-    int slow[16];
+    alignas(16) int slow[16];
     struct Grads {
         float Z[L][SP], Kh[L][SP], V[L][SP], SA[L][SP], S[NH][SP];
         float Ak[L][TP], Rk[L][TP], dAb[L][TP], dAk[L][TP], dRb[L][TP], dRk[L][TP];
@@ -106,9 +106,8 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
     constexpr int NW = kBwdThreads<GRADS> / 64;
     constexpr int CH = NH * L / kBwdThreads<GRADS>;       // channels per thread of the element-wise phases
     constexpr int TPW = L / NW;                           // tokens per wave there
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     typedef typename std::conditional<FI, double, float>::type DT;
-    BwdLds<GRADS, DT>& sm = *reinterpret_cast<BwdLds<GRADS, DT>*>(smem);
+    __shared__ BwdLds<GRADS, DT> sm;
     const int tid = threadIdx.x, lane0 = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int unit = blockIdx.x / nseg;
@@ -233,7 +232,10 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
         lds_barrier();
         int any_slow = 0;
 #pragma unroll
-        for (int q = 0; q < NW; ++q) any_slow |= sm.slow[q];
+        for (int q = 0; q < NW; q += 4) {
+            const int4 x = *reinterpret_cast<const int4*>(&sm.slow[q]);
+            any_slow |= x.x | x.y | x.z | x.w;
+        }
 
         if (any_slow) {
             // ---- exact token-serial update of the chunk.  Half 0 (512 threads): rows of G, thread (i, q)
@@ -355,13 +357,16 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
         DT before[CH];  // log2 D before this token
 #pragma unroll
         for (int e = 0; e < CH; ++e) before[e] = pre[e];
+        // (all reads first: a branch around each would wait for them one by one)
+        DT tots[NW - 1][CH];
 #pragma unroll
-        for (int q = 0; q < NW - 1; ++q) {
-            if (q < wave) {  // uniform
+        for (int q = 0; q < NW - 1; ++q)
 #pragma unroll
-                for (int e = 0; e < CH; ++e) before[e] += sm.tot[q][j0 + e];
-            }
-        }
+            for (int e = 0; e < CH; ++e) tots[q][e] = sm.tot[q][j0 + e];
+#pragma unroll
+        for (int q = 0; q < NW - 1; ++q)
+#pragma unroll
+            for (int e = 0; e < CH; ++e) before[e] += q < wave ? tots[q][e] : (DT)0;
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
             const DT ld = before[e] + lw2[e];
@@ -587,13 +592,15 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
                 for (int e = 0; e < CH; ++e) sm.tot[wave][j0 + e] = suf[e];
             }
             lds_barrier();
+            float sums[NW][CH];
 #pragma unroll
-            for (int q = 1; q < NW; ++q) {
-                if (q > wave) {  // uniform
+            for (int q = 1; q < NW; ++q)
 #pragma unroll
-                    for (int e = 0; e < CH; ++e) suf[e] += (float)sm.tot[q][j0 + e];
-                }
-            }
+                for (int e = 0; e < CH; ++e) sums[q][e] = (float)sm.tot[q][j0 + e];
+#pragma unroll
+            for (int q = 1; q < NW; ++q)
+#pragma unroll
+                for (int e = 0; e < CH; ++e) suf[e] += q > wave ? sums[q][e] : 0.f;
             const uint32_t o = (uint32_t)tk * stride + j0 * sizeof(IO);
 #pragma unroll
             for (int e = 0; e < CH; ++e) {
@@ -626,13 +633,26 @@ __global__ __launch_bounds__(kBwdThreads<GRADS>) void wkv7_train_bwd_chunk_kerne
     }
 }
 
-// Segments per unit: enough blocks for the 256 CUs (one block each), none shorter than a chunk.
+// Segments per unit, by the cost (us) of a walk's chunk: 9.6 in the gradient pass (one block per CU, rounds of
+// 256), 5.5 in the G pass (8 with two blocks on a CU; 2 n - 3 blocks per unit), 0.6 per step of the scan, and 30
+// for two more launches (12 on the device; the rest is what they cost a caller that enqueues as fast as it
+// can).  Measured (bf16, one segment -> split): 12 units of 96 tokens 33 -> 32 and not split,
+// of 512 tokens 158 -> 36, 64 units of 1,000 tokens 310 -> 140.
 int bwd_segments(int64_t units, int T, int* cps) {
     const int nchunk = (T + L - 1) / L;
-    int nseg = (int)(256 / units);
-    if (nseg > nchunk) nseg = nchunk;
-    if (nseg < 1) nseg = 1;
-    *cps = (nchunk + nseg - 1) / nseg;
+    *cps = nchunk;
+    if (units >= 256) return 1;
+    float best = 9.6f * nchunk;
+    for (int n = 2; n <= 64 && n <= nchunk; ++n) {
+        const int c = (nchunk + n - 1) / n, nn = (nchunk + c - 1) / c;
+        const int64_t b1 = units * (2 * nn - 3);
+        const float pass1 = b1 <= 256 ? 5.5f : 8.f * (float)((b1 + 511) / 512);
+        const float cost = c * (pass1 + 9.6f * (float)((units * nn + 255) / 256)) + 0.6f * nn + 30.f;
+        if (cost < best) {
+            best = cost;
+            *cps = c;
+        }
+    }
     return (nchunk + *cps - 1) / *cps;
 }
 
@@ -657,26 +677,21 @@ hipError_t launch_wkv7_train_bwd_chunk(int B, int T, int H, const void* r, const
     const int nseg = bwd_segments(units, T, &cps);
     float* q = ws;
     float* h = nseg > 1 ? ws + units * nseg * (NH * NH) : nullptr;
-    auto launch = [&](auto kern, dim3 grid, int threads, size_t lds) -> hipError_t {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, grid, dim3(threads), lds, st, T, H, nseg, cps, (const IO*)r, (const IO*)w, (const IO*)k,
+    auto launch = [&](auto kern, dim3 grid, int threads) -> hipError_t {
+        hipLaunchKernelGGL(kern, grid, dim3(threads), 0, st, T, H, nseg, cps, (const IO*)r, (const IO*)w, (const IO*)k,
                            (const IO*)v, (const IO*)a, (const IO*)b, (const IO*)dy, ckpt, sa, ds_in, s0, start_known,
                            q, h, (IO*)dr, (IO*)dw, (IO*)dk, (IO*)dv, (IO*)da, (IO*)db, ds0);
         return hipGetLastError();
     };
     const dim3 full((unsigned)(units * nseg)), two((unsigned)(units * nseg), 2);
-    typedef typename std::conditional<sizeof(IO) == 4, double, float>::type DT;
     auto passes = [&](auto exact) -> hipError_t {
         constexpr bool EX = decltype(exact)::value;
         if (nseg > 1) {
-            hipError_t e = launch(wkv7_train_bwd_chunk_kernel<IO, false, EX>, two, kBwdThreads<false>,
-                                  sizeof(BwdLds<false, DT>));
+            hipError_t e = launch(wkv7_train_bwd_chunk_kernel<IO, false, EX>, two, kBwdThreads<false>);
             if (e == hipSuccess && nseg > 2) e = launch_wkv7_scan_backward(units, nseg, q, h, st);
             if (e != hipSuccess) return e;
         }
-        return launch(wkv7_train_bwd_chunk_kernel<IO, true, EX>, full, kBwdThreads<true>, sizeof(BwdLds<true, DT>));
+        return launch(wkv7_train_bwd_chunk_kernel<IO, true, EX>, full, kBwdThreads<true>);
     };
     if constexpr (sizeof(IO) == 4) return passes(std::true_type());
     else return ds0 != nullptr ? passes(std::true_type()) : passes(std::false_type());
