@@ -50,6 +50,7 @@
 // MFMA operand layout (gfx950): lane l supplies row l%32 of A and of B, k =
 // 8*(l/32) .. +7; accumulator q of lane l is C[8*(q/4) + 4*(l/32) + q%4][l%32].
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "rwkv7_hip.h"
@@ -367,6 +368,82 @@ __global__ __launch_bounds__(T::THREADS) void gemm_decode_kernel(GemmBatch batch
         }
 }
 
+// Up to kFewRows rows (a token of one or a few interactive sequences): a block takes 16 weight rows of one
+// problem, or a K range of them, and its four waves every fourth 64-wide K tile.  A wave reads its weights
+// straight into the operand registers of v_mfma_f32_16x16x32_bf16 (lane l: row l % 16, 16-byte chunks l / 16 and
+// 4 + l / 16 of the packed tile's rows), the activation rows fill the 16 columns (clamped past M, not stored), and
+// kAheadTiles tiles are in flight per wave; the waves' sums meet in LDS.
+//
+// At these row counts a launch of the LDS-ring kernel is its own latency: the ring's fill, one barrier per stage
+// and, where K is split, the reduction launch; a 32 x 32 tile also gives a 768-wide projection only 24 blocks.
+// One row, 768-wide model (12 layers): launches of 5.8-6.8 us (x 5 per layer) -> 4.3-5.4 us and no
+// reduction launch; a step of 4 rows,
+// 4 layers of 1,024 channels 218 -> 193 us.
+constexpr int kFewRows = 7;
+constexpr int kAheadTiles = 4;
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) void gemm_few_kernel(GemmBatch batch, float* __restrict__ ws) {
+    __shared__ f32x4_t red[3][64];
+    const GemmProblem P = select_problem(batch, blockIdx.x, false);
+    const int M = batch.M;
+    const int local = blockIdx.x - P.block_begin;
+    const int ntile = local / P.splits, split = local - ntile * P.splits;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 15, h = lane >> 4;
+    const int n0 = 16 * ntile;
+    const int kt0 = split * P.k_per / BK, kt1 = min(P.k_tiles, kt0 + P.k_per / BK);
+    // this lane's row of the packed tiles and its two chunks there
+    const int r = (n0 & 63) + c;
+    const bf16_t* wrow = P.B + (int64_t)(n0 >> 6) * P.k_tiles * (64 * BK) + r * BK;
+    const int p0 = (h ^ swz(r)) * 8, p1 = ((4 + h) ^ swz(r)) * 8;
+    const bf16_t* xrow = P.A + (int64_t)min(c, M - 1) * P.lda;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    for (int t = kt0 + wave; t < kt1; t += 4 * kAheadTiles) {
+        uint4 w[kAheadTiles][2], x[kAheadTiles][2];
+#pragma unroll
+        for (int u = 0; u < kAheadTiles; ++u) {
+            const int kt = min(t + 4 * u, kt1 - 1);  // past the range: a tile whose products are left out
+            const bf16_t* wt = wrow + (int64_t)kt * (64 * BK);
+            w[u][0] = *reinterpret_cast<const uint4*>(wt + p0);
+            w[u][1] = *reinterpret_cast<const uint4*>(wt + p1);
+            // chunks past K: the weights there are zero, the activations must not be read
+            const int k0 = kt * BK + 8 * h, k1 = k0 + 32;
+            x[u][0] = *reinterpret_cast<const uint4*>(xrow + min(k0, P.K - 8));
+            x[u][1] = *reinterpret_cast<const uint4*>(xrow + min(k1, P.K - 8));
+            if (k0 >= P.K) x[u][0] = zero;
+            if (k1 >= P.K) x[u][1] = zero;
+        }
+#pragma unroll
+        for (int u = 0; u < kAheadTiles; ++u) {
+            if (t + 4 * u < kt1) {  // uniform
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[u][q]),
+                                                                  __builtin_bit_cast(bf16x8_t, x[u][q]), acc, 0, 0, 0);
+            }
+        }
+    }
+    if (wave > 0) red[wave - 1][lane] = acc;
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) acc += red[q][lane];
+    // element e: weight row n0 + 4 h + e, activation row c
+    if (c >= M) return;
+    const int n = n0 + 4 * h;
+    const bool planes = P.splits > 1 || P.partial;
+    float* part = ws + P.ws_off + ((int64_t)split * M + c) * P.N;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= P.N) break;
+        if (planes) part[n + e] = acc[e];
+        else P.C[(int64_t)c * P.ldc + n + e] = f32_to_bf16(epi_fn(P.epi, acc[e]));
+    }
+}
+
 // Sum the split-K partials in split order (deterministic), apply the epilogue
 // and write bf16.  Thread e of problem p covers 4 consecutive elements of the
 // problem's [M][N] partial rows; red_begin is the problem's first block here.
@@ -449,10 +526,42 @@ Plan make_plan(int bm, int bn, int M, int count, const int* N, const int* K, int
     return pl;
 }
 
+// The same for gemm_few_kernel: 16-row column tiles, no rows tiles.
+Plan few_plan(int M, int count, const int* N, const int* K, bool partial) {
+    // results with an epilogue: split (with the reduction launch) only where a handful of blocks would be left;
+    // partial planes cost a few rows' reads in the next kernel: about one block per CU
+    const int target = partial ? 256 : 32, min_k = partial ? 256 : 512;
+    Plan pl{};
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) total += (N[i] + 15) / 16;
+    for (int i = 0; i < count; ++i) {
+        int si = (int)((target + total - 1) / total);
+        if (si > K[i] / min_k) si = K[i] / min_k;
+        if (si > 8) si = 8;
+        if (si < 1) si = 1;
+        int kp = (K[i] + si - 1) / si;
+        kp = (kp + BK - 1) / BK * BK;
+        si = (K[i] + kp - 1) / kp;
+        pl.splits[i] = si;
+        pl.k_per[i] = kp;
+        pl.blocks += (N[i] + 15) / 16 * si;
+        if (si > 1) {
+            pl.ws_floats += (int64_t)si * M * N[i];
+            pl.red_tiles += (int)((((int64_t)M * N[i] + 3) / 4 + 255) / 256);
+        }
+    }
+    return pl;
+}
+
+struct FewTile {
+    static constexpr int BM = kFewRows, BN = 16, THREADS = 256;
+};
+
 template <class T>
 hipError_t launch_tile(int M, int count, const void* const* A, const void* const* B, void* const* C,
                        const int64_t* lda, const int64_t* ldc, const int* N, const int* K,
                        const int* epi, float* ws, hipStream_t st, const Plan& pl, int partial = 0) {
+    constexpr bool few = std::is_same<T, FewTile>::value;
     GemmBatch b{};
     b.count = count;
     b.M = M;
@@ -479,14 +588,15 @@ hipError_t launch_tile(int M, int count, const void* const* A, const void* const
         p.block_begin = blocks;
         p.ws_off = ws_off;
         p.red_begin = red;
-        blocks += 8 * ((p.n_tiles + 7) / 8) * mt * p.splits;
+        blocks += few ? p.n_tiles * p.splits : 8 * ((p.n_tiles + 7) / 8) * mt * p.splits;
         p.partial = partial;
         if (p.splits > 1 || partial) {
             ws_off += (int64_t)p.splits * M * N[i];
             if (!partial) red += (int)((((int64_t)M * N[i] + 3) / 4 + 255) / 256);
         }
     }
-    hipLaunchKernelGGL((gemm_decode_kernel<T>), dim3(blocks), dim3(T::THREADS), 0, st, b, ws);
+    if constexpr (few) hipLaunchKernelGGL(gemm_few_kernel, dim3(blocks), dim3(T::THREADS), 0, st, b, ws);
+    else hipLaunchKernelGGL((gemm_decode_kernel<T>), dim3(blocks), dim3(T::THREADS), 0, st, b, ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || red == 0 || partial) return e;
     hipLaunchKernelGGL(gemm_reduce_kernel, dim3(red), dim3(256), 0, st, b, (const float*)ws);
@@ -497,6 +607,8 @@ hipError_t launch_tile(int M, int count, const void* const* A, const void* const
 // 256 x 32, 64 x 64, 128 x 64; 4 to 16 waves) and block targets (1 to 512)
 // over the five launches of a 1.5B and a 7.2B decode layer at M = 32 .. 256,
 // cold weights (MI355X; the plans compared in one process, interleaved):
+//   * up to 7 rows the latency-bound kernel without a ring (gemm_few_kernel); 8 rows and more, the smallest
+//     row buckets of a rollout, give the bits of the 32-row plan;
 //   * up to 32 rows a 32 x 32 tile (4 K groups) with K split to about 256
 //     blocks (summed by the reduction launch): every block only streams
 //     weights, and the narrow tile gives twice the column tiles and half the
@@ -523,7 +635,7 @@ using TileDecode = Tile<2, 2, 1, 1, 4, 2>;
 using TileWide = Tile<4, 2, 1, 1, 4, 1>;
 constexpr int kMinK = 512;
 
-enum TileKind { kNarrow, kDecode, kWide };
+enum TileKind { kNarrow, kDecode, kWide, kFew };
 
 // compute units of the current device (queried once per device)
 int cu_count() {
@@ -541,6 +653,7 @@ int cu_count() {
 }
 
 TileKind tile_for(int M, bool partial, int count, const int* N) {
+    if (M <= kFewRows) return kFew;
     if (M <= 32) return kNarrow;
     if (partial) return M <= 64 ? kDecode : kWide;
     const int cus = cu_count();
@@ -568,6 +681,7 @@ int target_for(int M, bool partial) {
 Plan plan_for(int M, int count, const int* N, const int* K, bool partial) {
     const int target = target_for(M, partial);
     switch (tile_for(M, partial, count, N)) {
+        case kFew: return few_plan(M, count, N, K, partial);
         case kNarrow: return make_plan(TileNarrow::BM, TileNarrow::BN, M, count, N, K, target, kMinK, 0);
         case kDecode: return make_plan(TileDecode::BM, TileDecode::BN, M, count, N, K, target, kMinK, 0);
         default: return make_plan(TileWide::BM, TileWide::BN, M, count, N, K, target, kMinK, 0);
@@ -579,6 +693,7 @@ hipError_t launch_for(int M, int count, const void* const* A, const void* const*
                       hipStream_t st, int partial) {
     const Plan pl = plan_for(M, count, N, K, partial != 0);
     switch (tile_for(M, partial != 0, count, N)) {
+        case kFew: return launch_tile<FewTile>(M, count, A, B, C, lda, ldc, N, K, epi, ws, st, pl, partial);
         case kNarrow: return launch_tile<TileNarrow>(M, count, A, B, C, lda, ldc, N, K, epi, ws, st, pl, partial);
         case kDecode: return launch_tile<TileDecode>(M, count, A, B, C, lda, ldc, N, K, epi, ws, st, pl, partial);
         default: return launch_tile<TileWide>(M, count, A, B, C, lda, ldc, N, K, epi, ws, st, pl, partial);
